@@ -150,6 +150,19 @@ int nvx_temperature_softmax(const void* logits, int32_t logits_dtype, int64_t lo
                             const float* temperatures, float* probs, int32_t num_rows,
                             int32_t vocab, void* stream);
 
+/* ------------------------------------------------------------- sampled tokens --
+ * One token per row (reference nanovllm/layers/sampler.py:5-12): the categorical draw of
+ * softmax(float(logits[r]) / temperatures[r]) by inverse CDF with uniforms[r], or the
+ * first index of the largest logit where temperatures[r] == 0.  The token is the one
+ * nvx_temperature_softmax followed by nvx_rejection_sample_tree (one node, draft_mode 1)
+ * gives, without the probabilities in memory; -1 for a row with no positive probability.
+ *   logits as in nvx_temperature_softmax   uniforms fp32 [num_rows]
+ *   tokens int64 [num_rows]                vocab <= 2,097,152
+ */
+int nvx_sample(const void* logits, int32_t logits_dtype, int64_t logits_row_stride,
+               const float* temperatures, const float* uniforms, int64_t* tokens,
+               int32_t num_rows, int32_t vocab, void* stream);
+
 /* -------------------------------------------------- tree rejection sampling --
  * Verifies one draft tree per sequence and emits the accepted path plus one
  * recovered/bonus token.  Sits beside Sampler.forward (reference

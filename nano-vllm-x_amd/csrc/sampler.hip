@@ -51,6 +51,58 @@ __device__ __forceinline__ float load_logit(const void* row, int i, int dtype) {
 // keeps the relative error ~1e-6 (contract tolerance 1e-5).
 constexpr int kVecNT = 1024;
 
+// The statistics pass: online max and sum over the nvec 16-byte vectors of a row, kU
+// loads in flight per thread.  The order of the sums is part of a softmax's bits (kU
+// decides which values share a partial sum).  kNt: non-temporal loads.
+template <typename VT, int kU, bool kNt>
+__device__ __forceinline__ void vec_row_stats(const uint4* __restrict__ src, int nvec, float a,
+                                              float* red, float* M, float* inv) {
+  using Tr = nvx::VecTraits<VT>;
+  constexpr int P = Tr::kPer;
+  float m = -INFINITY, s = 0.f;
+  int i = threadIdx.x;
+  for (; i + (kU - 1) * kVecNT < nvec; i += kU * kVecNT) {
+    uint4 w[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      w[u] = kNt ? nvx::ld_stream(src + i + u * kVecNT) : src[i + u * kVecNT];
+    float lm = -INFINITY;
+    float x[kU][P];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      Tr::expand(w[u], x[u]);
+#pragma unroll
+      for (int e = 0; e < P; ++e) lm = fmaxf(lm, x[u][e]);
+    }
+    const float mn = fmaxf(m, lm * a);
+    if (mn == -INFINITY) continue;  // every value so far is -inf
+    float acc = 0.f;
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int e = 0; e < P; ++e) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(x[u][e], a, -mn));
+    s = (m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f(m - mn)) + acc;
+    m = mn;
+  }
+  for (; i < nvec; i += kVecNT) {
+    float x[P];
+    Tr::expand(src[i], x);
+    float lm = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < P; ++e) lm = fmaxf(lm, x[e]);
+    const float mn = fmaxf(m, lm * a);
+    if (mn == -INFINITY) continue;
+    float acc = 0.f;
+#pragma unroll
+    for (int e = 0; e < P; ++e) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], a, -mn));
+    s = (m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f(m - mn)) + acc;
+    m = mn;
+  }
+  *M = nvx::block_max<kVecNT>(m, red);
+  const float part = (m == -INFINITY) ? 0.f : s * __builtin_amdgcn_exp2f(m - *M);
+  *inv = 1.f / nvx::block_sum_any<kVecNT>(part, red);
+}
+
 // Modes of the streaming kernel.  kSoftmax: both passes.  kStatsOnly: the first pass
 // only; stores (max in log2 units, 1/sum) for the row in stats[row] (the fused
 // rejection walk recomputes each probability it reads).  kFromStats: the second pass
@@ -94,47 +146,7 @@ __global__ __launch_bounds__(kVecNT) void softmax_vec_kernel(const VT* __restric
     M = stats[row].x;
     inv = stats[row].y;
   } else {
-    float m = -INFINITY, s = 0.f;
-    for (; i + (kUnroll - 1) * kVecNT < nvec; i += kUnroll * kVecNT) {
-      uint4 w[kUnroll];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
-        w[u] = kMode == kStatsOnly ? nvx::ld_stream(src + i + u * kVecNT) : src[i + u * kVecNT];
-      float lm = -INFINITY;
-      float x[kUnroll][P];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        Tr::expand(w[u], x[u]);
-#pragma unroll
-        for (int e = 0; e < P; ++e) lm = fmaxf(lm, x[u][e]);
-      }
-      const float mn = fmaxf(m, lm * a);
-      if (mn == -INFINITY) continue;  // every value so far is -inf
-      float acc = 0.f;
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
-#pragma unroll
-        for (int e = 0; e < P; ++e) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(x[u][e], a, -mn));
-      s = (m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f(m - mn)) + acc;
-      m = mn;
-    }
-    for (; i < nvec; i += kVecNT) {
-      float x[P];
-      Tr::expand(src[i], x);
-      float lm = -INFINITY;
-#pragma unroll
-      for (int e = 0; e < P; ++e) lm = fmaxf(lm, x[e]);
-      const float mn = fmaxf(m, lm * a);
-      if (mn == -INFINITY) continue;
-      float acc = 0.f;
-#pragma unroll
-      for (int e = 0; e < P; ++e) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], a, -mn));
-      s = (m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f(m - mn)) + acc;
-      m = mn;
-    }
-    M = nvx::block_max<kVecNT>(m, red);
-    const float part = (m == -INFINITY) ? 0.f : s * __builtin_amdgcn_exp2f(m - M);
-    inv = 1.f / nvx::block_sum_any<kVecNT>(part, red);
+    vec_row_stats<VT, kU, kMode == kStatsOnly>(src, nvec, a, red, &M, &inv);
     if constexpr (kMode == kStatsOnly) {
       if (tid == 0) stats[row] = make_float2(M, inv);
       return;
@@ -186,6 +198,64 @@ __global__ __launch_bounds__(kVecNT) void softmax_vec_kernel(const VT* __restric
 constexpr int kRegNT = 512;
 
 template <int NG>
+struct RegRow {
+  using Tr = nvx::VecTraits<uint16_t>;
+  uint4 w[NG];
+  bool tail_ok;
+  __device__ __forceinline__ RegRow(const uint16_t* row, int V) {
+    constexpr int kRsrcWord3 = 0x00020000;  // gfx9 buffer descriptor word 3 (raw dword access)
+    const __amdgpu_buffer_rsrc_t in_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(row), 0, V * 2, kRsrcWord3);
+    const int tid = threadIdx.x;
+    const int voff = tid * 16;
+    tail_ok = tid + (NG - 1) * kRegNT < V / 8;
+#pragma unroll
+    for (int u = 0; u < NG - 1; ++u)
+      w[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(in_rsrc, voff, u * kRegNT * 16, 0));
+    w[NG - 1] = make_uint4(0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u);  // bf16 -inf
+    if (tail_ok)
+      w[NG - 1] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(in_rsrc, voff, (NG - 1) * kRegNT * 16, 0));
+  }
+  // Each pass re-expands from the packed registers: without this the compiler keeps
+  // the expanded fp32 values of the first pass live (8 bytes per two logits).
+  __device__ __forceinline__ void opaque() {
+#pragma unroll
+    for (int u = 0; u < NG; ++u)
+      asm volatile("" : "+v"(w[u].x), "+v"(w[u].y), "+v"(w[u].z), "+v"(w[u].w));
+  }
+  // This thread's largest logit.
+  __device__ __forceinline__ float lane_max() const {
+    float lm = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < NG; ++u) {
+      float x[8];
+      Tr::expand(w[u], x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) lm = fmaxf(lm, x[e]);
+    }
+    return lm;
+  }
+  // Row max in log2 units (a = log2(e) / T) and 1 / sum.
+  __device__ __forceinline__ void stats(float a, float* red, float* M, float* inv) {
+    *M = nvx::block_max<kRegNT>(lane_max() * a, red);
+    opaque();
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+    for (int u = 0; u < NG; ++u) {
+      float x[8];
+      Tr::expand(w[u], x);
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        s0 += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], a, -*M));
+        s1 += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e + 1], a, -*M));
+      }
+    }
+    *inv = 1.f / nvx::block_sum_any<kRegNT>(s0 + s1, red);
+  }
+};
+
+template <int NG>
 __global__ __launch_bounds__(kRegNT) void softmax_row_kernel(const uint16_t* __restrict__ logits,
                                                              int64_t stride,
                                                              const float* __restrict__ temps,
@@ -207,58 +277,20 @@ __global__ __launch_bounds__(kRegNT) void softmax_row_kernel(const uint16_t* __r
     }
     return;
   }
-  constexpr int kRsrcWord3 = 0x00020000;  // gfx9 buffer descriptor word 3 (raw dword access)
-  const __amdgpu_buffer_rsrc_t in_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(logits + (int64_t)row * stride), 0, V * 2, kRsrcWord3);
-  const int voff = tid * 16;
-  const bool tail_ok = tid + (NG - 1) * kRegNT < nvec;
-  uint4 w[NG];
-#pragma unroll
-  for (int u = 0; u < NG - 1; ++u)
-    w[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(in_rsrc, voff, u * kRegNT * 16, 0));
-  w[NG - 1] = make_uint4(0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u);  // bf16 -inf
-  if (tail_ok)
-    w[NG - 1] = __builtin_bit_cast(
-        uint4, __builtin_amdgcn_raw_buffer_load_b128(in_rsrc, voff, (NG - 1) * kRegNT * 16, 0));
+  RegRow<NG> r(logits + (int64_t)row * stride, V);
+  uint4(&w)[NG] = r.w;
   float* const out_row = probs + (int64_t)row * V;
   auto store = [&](int u, const float (&y)[8]) {
-    if (u < NG - 1 || tail_ok) {
+    if (u < NG - 1 || r.tail_ok) {
       float* d = out_row + (uint32_t)(tid * 8 + u * kRegNT * 8);
       *reinterpret_cast<float4*>(d) = make_float4(y[0], y[1], y[2], y[3]);
       *reinterpret_cast<float4*>(d + 4) = make_float4(y[4], y[5], y[6], y[7]);
     }
   };
-  // Each pass re-expands from the packed registers: without this the compiler keeps
-  // the expanded fp32 values of the first pass live (8 bytes per two logits).
-  auto opaque = [&]() {
-#pragma unroll
-    for (int u = 0; u < NG; ++u)
-      asm volatile("" : "+v"(w[u].x), "+v"(w[u].y), "+v"(w[u].z), "+v"(w[u].w));
-  };
   const float a = 1.4426950408889634f / T;
-  float lm = -INFINITY;
-#pragma unroll
-  for (int u = 0; u < NG; ++u) {
-    float x[8];
-    Tr::expand(w[u], x);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) lm = fmaxf(lm, x[e]);
-  }
-  const float M = nvx::block_max<kRegNT>(lm * a, red);
-  opaque();
-  float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-  for (int u = 0; u < NG; ++u) {
-    float x[8];
-    Tr::expand(w[u], x);
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      s0 += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], a, -M));
-      s1 += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e + 1], a, -M));
-    }
-  }
-  const float inv = 1.f / nvx::block_sum_any<kRegNT>(s0 + s1, red);
-  opaque();
+  float M, inv;
+  r.stats(a, red, &M, &inv);
+  r.opaque();
 #pragma unroll
   for (int u = 0; u < NG; ++u) {
     float x[8];
@@ -274,6 +306,26 @@ __global__ __launch_bounds__(kRegNT) void softmax_row_kernel(const uint16_t* __r
 inline int row_kernel_groups(int vocab) { return (vocab / 8 + kRegNT - 1) / kRegNT; }
 
 // --------------------------------------------------------- softmax (stream)
+// Online max / sum over the raw logits in log2 units (x * a, a = log2(e) / T), one value
+// per load.
+__device__ __forceinline__ void stream_row_stats(const void* src, int dtype, int V, float a,
+                                                 float* red, float* M, float* inv) {
+  float m = -INFINITY, s = 0.f;
+  for (int i = threadIdx.x; i < V; i += kNT) {
+    const float x = load_logit(src, i, dtype) * a;
+    if (x == -INFINITY) continue;
+    if (x > m) {
+      s = s * __builtin_amdgcn_exp2f(m - x) + 1.f;
+      m = x;
+    } else {
+      s += __builtin_amdgcn_exp2f(x - m);
+    }
+  }
+  *M = nvx::block_max<kNT>(m, red);
+  const float part = (m == -INFINITY) ? 0.f : s * __builtin_amdgcn_exp2f(m - *M);
+  *inv = 1.f / nvx::block_sum_any<kNT>(part, red);
+}
+
 __global__ __launch_bounds__(kNT) void softmax_stream_kernel(const void* __restrict__ logits,
                                                              int dtype, int64_t stride,
                                                              const float* __restrict__ temps,
@@ -289,22 +341,9 @@ __global__ __launch_bounds__(kNT) void softmax_stream_kernel(const void* __restr
     for (int i = threadIdx.x; i < V; i += kNT) dst[i] = load_logit(src, i, dtype);
     return;
   }
-  // Online max / sum over the raw logits in log2 units (x * log2(e) / T).
   const float a = 1.4426950408889634f / T;
-  float m = -INFINITY, s = 0.f;
-  for (int i = threadIdx.x; i < V; i += kNT) {
-    const float x = load_logit(src, i, dtype) * a;
-    if (x == -INFINITY) continue;
-    if (x > m) {
-      s = s * __builtin_amdgcn_exp2f(m - x) + 1.f;
-      m = x;
-    } else {
-      s += __builtin_amdgcn_exp2f(x - m);
-    }
-  }
-  const float M = nvx::block_max<kNT>(m, red);
-  const float part = (m == -INFINITY) ? 0.f : s * __builtin_amdgcn_exp2f(m - M);
-  const float inv = 1.f / nvx::block_sum_any<kNT>(part, red);
+  float M, inv;
+  stream_row_stats(src, dtype, V, a, red, &M, &inv);
   for (int i = threadIdx.x; i < V; i += kNT)
     dst[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(load_logit(src, i, dtype), a, -M)) * inv;
 }
@@ -1146,6 +1185,211 @@ void rejection_walk_kernel(Src src, WalkArgs a) {
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// ------------------------------------------------------- one draw per row
+// nvx_sample: temperature softmax and categorical draw of each logits row in one
+// launch, without writing probabilities.  One workgroup per row: the row statistics
+// (the pass nvx_temperature_softmax makes for the same row), then the walk's
+// inverse-CDF draw (one node, no children) on probabilities recomputed from the logits
+// as exp2(fma(x, log2(e)/T, -max)) * (1/sum); rows at temperature 0 take the first index
+// of their largest logit.  The sums, chains and the pick associate exactly as
+// nvx_temperature_softmax followed by the walk, so the tokens are the same.
+//
+// Bound by the exponentials (two per logit at a quarter of the VALU rate: ~8 us of a
+// 151,936-logit row's CU) and the row's two reads (HBM, then the Infinity Cache).
+// [256, 151936] bf16: 32.7 us per call; softmax, walk and the seven small launches
+// around them took 122 us (155 MB of fp32 probabilities written and read back).
+constexpr int kLanePitch = kLW + 1;    // lane sums of a logical wave in LDS, padded
+
+struct DrawShared {
+  float lanes[kLW * kLanePitch];  // lane sums, then lane chains, of the 64 logical waves
+  float wpre[kLW];                // row chain: sum of the logical waves before
+  float total;
+  float red[kNW];
+  int redi[kNW + 1];
+};
+
+// The draw of chain_pass + chain_pick<kPlain> by one workgroup of NT threads.  Each
+// lane's sums of the 64 logical waves meet in LDS, where one wave chains all of them at
+// once (lane w chains logical wave w), instead of 64 / NW chains in turn on every wave.
+template <int NT, typename PRow>
+__device__ int draw_row(const PRow& row, int V, bool vec, float u, DrawShared& sh) {
+  constexpr int NW = NT / 64, M = kLW / NW;
+  constexpr int kDrawBatch = sizeof(typename PRow::Raw) == 16 ? 10 : 5;  // subtiles' loads in flight
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Layout lay(V);
+  const PassSpec ps{kPlain, 0.f, nullptr, 0};
+  const int lw0 = wave * M;
+  const int jlo = lay.lo(lw0), jhi = lay.hi(lw0 + M - 1);
+  const int jfull = vec ? max(jlo, min(jhi, V / kSub)) : jlo;
+  int lw = lw0, jend = lay.hi(lw0);
+  float L = 0.f;
+  auto close = [&](int j) {  // subtiles before j are done: finish the logical waves they end
+    while (lw < lw0 + M && j >= jend) {
+      sh.lanes[lw * kLanePitch + lane] = L;
+      L = 0.f;
+      ++lw;
+      jend = lay.hi(lw);
+    }
+  };
+  close(jlo);
+  for (int jb = jlo; jb < jfull; jb += kDrawBatch) {
+    typename PRow::Raw pr[kDrawBatch];
+#pragma unroll
+    for (int t = 0; t < kDrawBatch; ++t)
+      if (jb + t < jfull) pr[t] = row.fetch((jb + t) * kSub + lane * 8);
+#pragma unroll
+    for (int t = 0; t < kDrawBatch; ++t) {
+      if (jb + t < jfull) {
+        float v[8];
+        row.values(pr[t], v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) L = L + v[e];
+        close(jb + t + 1);
+      }
+    }
+  }
+  for (int j = jfull; j < jhi; ++j) {
+    float v[8];
+    row.load8(j * kSub + lane * 8, V, vec, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) L = L + v[e];
+    close(j + 1);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float* mine = sh.lanes + lane * kLanePitch;
+    float run = 0.f;
+#pragma unroll 16
+    for (int l = 0; l < 64; ++l) {
+      run = run + mine[l];
+      mine[l] = run;
+    }
+    float tot = 0.f, W = 0.f;
+#pragma unroll
+    for (int l = 0; l < 64; ++l) {
+      W = lane == l ? tot : W;
+      tot = tot + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(run), l));
+    }
+    sh.wpre[lane] = W;
+    if (lane == 0) sh.total = tot;
+  }
+  __syncthreads();
+  const float tau = u * sh.total;
+  int cand = INT32_MAX;
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    const uint64_t m = __ballot((sh.wpre[lw0 + i] + sh.lanes[(lw0 + i) * kLanePitch + lane]) > tau);
+    if (cand == INT32_MAX && m) cand = (lw0 + i) * 64 + __ffsll((unsigned long long)m) - 1;
+  }
+  const int gstar = nvx::block_min_i<NT>(cand, sh.redi);
+  if (gstar == INT32_MAX) {  // u * total rounds to the total (or is NaN)
+    int last = -1;
+    for (int j = jlo; j < jhi; ++j) {
+      float v[8];
+      residual8(row, nullptr, j * kSub + lane * 8, V, vec, false, ps, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (v[e] > 0.f) last = j * kSub + lane * 8 + e;
+    }
+    return nvx::block_max_i<NT>(last, sh.redi);
+  }
+  const int glw = gstar / 64, l = gstar % 64;
+  if (wave == 0) {
+    const float w_start = sh.wpre[glw];
+    float run = l > 0 ? w_start + sh.lanes[glw * kLanePitch + l - 1] : w_start;
+    const int j0 = lay.lo(glw), nk = lay.hi(glw) - j0;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (lane < nk) row.load8((j0 + lane) * kSub + l * 8, V, vec, v);
+    int first = -1, last = -1;
+    for (int kk = 0; kk < nk; ++kk) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[e]), kk));
+        run = run + x;
+        if (x > 0.f) {
+          const int y = (j0 + kk) * kSub + l * 8 + e;
+          if (first < 0 && run > tau) first = y;
+          last = y;
+        }
+      }
+    }
+    if (lane == 0) sh.redi[NW] = first >= 0 ? first : last;
+  }
+  __syncthreads();
+  return sh.redi[NW];
+}
+
+// First index of the row's largest logit (0 when every logit is NaN).
+template <int NT, typename VT>
+__device__ int argmax_row(const VT* logits, int V, bool vec, DrawShared& sh) {
+  using Tr = nvx::VecTraits<VT>;
+  constexpr int P = Tr::kPer, kU = 8;
+  const int nvec = vec ? V / P : 0;
+  const uint4* src = reinterpret_cast<const uint4*>(logits);
+  float bv = -INFINITY;
+  int bi = INT32_MAX;
+  // a thread's indices ascend, so only a larger value replaces its first best
+  auto take = [&](float x, int y) {
+    if (x > bv || (x == bv && bi == INT32_MAX)) {
+      bv = x;
+      bi = y;
+    }
+  };
+  for (int i = threadIdx.x; i < nvec; i += kU * NT) {
+    uint4 w[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (i + u * NT < nvec) w[u] = nvx::ld_stream(src + i + u * NT);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (i + u * NT < nvec) {
+        float x[P];
+        Tr::expand(w[u], x);
+#pragma unroll
+        for (int e = 0; e < P; ++e) take(x[e], (i + u * NT) * P + e);
+      }
+    }
+  }
+  for (int y = nvec * P + threadIdx.x; y < V; y += NT) take(LogitRow<VT>::val(logits, y), y);
+  const float best = nvx::block_max<NT>(bv, sh.red);
+  const int r = nvx::block_min_i<NT>(bv == best ? bi : INT32_MAX, sh.redi);
+  return r == INT32_MAX ? 0 : r;
+}
+
+// Sources of a row's statistics: the three softmax kernels' passes.
+enum { kDrawRegs38 = 0, kDrawRegs32 = 1, kDrawVec = 2, kDrawStream = 3 };
+
+template <typename VT, int kStats>
+__global__ __launch_bounds__(kStats <= kDrawRegs32 ? kRegNT : kVecNT)
+void sample_kernel(const VT* __restrict__ logits, int64_t stride, const float* __restrict__ temps,
+                   const float* __restrict__ uniforms, int64_t* __restrict__ out, int V) {
+  constexpr int NT = kStats <= kDrawRegs32 ? kRegNT : kVecNT;
+  constexpr bool vec = kStats != kDrawStream;
+  __shared__ DrawShared sh;
+  const VT* row = logits + (int64_t)blockIdx.x * stride;
+  const float T = temps[blockIdx.x];
+  int token;
+  if (T == 0.f) {
+    token = argmax_row<NT, VT>(row, V, vec, sh);
+  } else {
+    const float a = 1.4426950408889634f / T;
+    float M, inv;
+    if constexpr (kStats == kDrawRegs38) {
+      RegRow<38>(reinterpret_cast<const uint16_t*>(row), V).stats(a, sh.red, &M, &inv);
+    } else if constexpr (kStats == kDrawRegs32) {
+      RegRow<32>(reinterpret_cast<const uint16_t*>(row), V).stats(a, sh.red, &M, &inv);
+    } else if constexpr (kStats == kDrawVec) {
+      vec_row_stats<VT, 8, false>(reinterpret_cast<const uint4*>(row), V / nvx::VecTraits<VT>::kPer, a,
+                                  sh.red, &M, &inv);
+    } else {
+      stream_row_stats(row, sizeof(VT) == 2 ? NVX_DTYPE_BF16 : NVX_DTYPE_F32, V, a, sh.red, &M, &inv);
+    }
+    token = draw_row<NT>(LogitRow<VT>{row, a, M, inv, false}, V, vec, uniforms[blockIdx.x], sh);
+  }
+  if (threadIdx.x == 0) out[blockIdx.x] = token;
+}
+
 // Workgroups a device holds at once of rejection_walk_kernel<Src, K> (0 if unknown),
 // cached per device.
 template <typename Src, int K>
@@ -1277,6 +1521,42 @@ extern "C" int nvx_temperature_softmax(const void* logits, int32_t logits_dtype,
     hipLaunchKernelGGL(softmax_stream_kernel, dim3(num_rows), dim3(kNT), 0, s, logits, logits_dtype,
                        logits_row_stride, temperatures, probs, vocab);
   }
+  NVX_LAUNCHED();
+  return NVX_OK;
+}
+
+// The statistics pass matches nvx_temperature_softmax's choice for the same rows (its
+// probability rows are always 16-byte aligned there when vocab allows), since the pass
+// decides the bits of the statistics.
+extern "C" int nvx_sample(const void* logits, int32_t logits_dtype, int64_t logits_row_stride,
+                          const float* temperatures, const float* uniforms, int64_t* tokens,
+                          int32_t num_rows, int32_t vocab, void* stream) {
+  nvx::clear_error();
+  NVX_CHECK(logits_dtype == NVX_DTYPE_F32 || logits_dtype == NVX_DTYPE_BF16,
+            "sample: logits must be fp32 or bf16 (dtype code %d)", logits_dtype);
+  NVX_CHECK(num_rows >= 0 && vocab >= 1 && logits_row_stride >= vocab,
+            "sample: bad sizes (rows=%d, vocab=%d, stride=%lld)", num_rows, vocab,
+            (long long)logits_row_stride);
+  if (num_rows == 0) return NVX_OK;
+  NVX_CHECK(logits && temperatures && uniforms && tokens, "sample: null pointer");
+  NVX_CHECK(vocab <= kMaxVocab, "sample: vocab %d exceeds %d", vocab, kMaxVocab);
+  hipStream_t s = (hipStream_t)stream;
+  nvx::TimerScope timer(NVX_TIMER_SOFTMAX, s);
+  const bool bf16 = logits_dtype == NVX_DTYPE_BF16;
+  const int per = bf16 ? 8 : 4;
+  const bool vec = vocab % per == 0 && logits_row_stride % per == 0 && aligned16(logits);
+  const int groups = row_kernel_groups(vocab);
+  const dim3 grid(num_rows);
+#define NVX_SAMPLE(VT, KIND, NT)                                                              \
+  hipLaunchKernelGGL((sample_kernel<VT, KIND>), grid, dim3(NT), 0, s, (const VT*)logits,      \
+                     logits_row_stride, temperatures, uniforms, tokens, vocab)
+  if (vec && bf16 && groups == 38) NVX_SAMPLE(uint16_t, kDrawRegs38, kRegNT);
+  else if (vec && bf16 && groups == 32) NVX_SAMPLE(uint16_t, kDrawRegs32, kRegNT);
+  else if (vec && bf16) NVX_SAMPLE(uint16_t, kDrawVec, kVecNT);
+  else if (vec) NVX_SAMPLE(float, kDrawVec, kVecNT);
+  else if (bf16) NVX_SAMPLE(uint16_t, kDrawStream, kVecNT);
+  else NVX_SAMPLE(float, kDrawStream, kVecNT);
+#undef NVX_SAMPLE
   NVX_LAUNCHED();
   return NVX_OK;
 }

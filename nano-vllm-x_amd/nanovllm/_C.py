@@ -38,6 +38,8 @@ _SIGS = {
                                     c_void_p], c_int32),
     "nvx_temperature_softmax": ([c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_int32, c_int32,
                                  c_void_p], c_int32),
+    "nvx_sample": ([c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_int32, c_int32,
+                    c_void_p], c_int32),
     "nvx_rejection_sample_tree": ([c_void_p, c_int64, c_void_p, c_int64, c_int32, c_void_p,
                                    c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
                                    c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,

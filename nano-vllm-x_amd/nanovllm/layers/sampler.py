@@ -312,15 +312,23 @@ class Sampler(nn.Module):
     """Sampler()(logits [N, V], temperatures [N]) -> int64 token ids [N]."""
 
     def forward(self, logits: torch.Tensor, temperatures: torch.Tensor, uniforms=None):
+        if logits.dim() != 2 or logits.stride(1) != 1:
+            raise ValueError("Sampler: logits must be [N, V] with unit stride in V")
+        if logits.dtype not in _DTYPE_CODE:
+            raise ValueError(f"Sampler: unsupported logits dtype {logits.dtype}")
         N, V = logits.shape
-        probs = temperature_softmax(logits, temperatures)
         dev = logits.device
-        u = torch.rand(N, device=dev) if uniforms is None else uniforms
-        zeros = torch.zeros(N, 1, dtype=torch.int32, device=dev)
-        greedy = temperatures.to(dev) == 0
-        _, _, _, nxt = rejection_sample_tree(probs.view(N, 1, V), None, zeros, zeros - 1,
-                                             zeros.float(), u, greedy, draft_mode="delta")
-        return nxt.long()
+        temps = temperatures.to(device=dev, dtype=torch.float32).contiguous()
+        u = torch.rand(N, device=dev) if uniforms is None else \
+            uniforms.to(torch.float32).contiguous()
+        if temps.numel() != N or u.numel() < N:
+            raise ValueError("Sampler: one temperature and one uniform per row")
+        tokens = torch.empty(N, dtype=torch.int64, device=dev)
+        _C.require_cuda(logits, temps, u)
+        _C.check(_C.lib().nvx_sample(
+            _C.ptr(logits), _DTYPE_CODE[logits.dtype], logits.stride(0), _C.ptr(temps), _C.ptr(u),
+            _C.ptr(tokens), N, V, _C.stream_of(logits)))
+        return tokens
 
 
 class RejectionSampler(nn.Module):

@@ -487,3 +487,41 @@ def test_fused_sampler_verify8b_batch(dev, delta):
     del P, two
     check_lazy(logits, row_temps, stats, args, greedy, None if delta else Q.cpu().numpy(),
                toks.cpu().numpy(), parents, U.cpu().numpy(), Uf.cpu().numpy(), delta)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,V,pad", [(1, 1, 0), (3, 7, 0), (2, 511, 1), (5, 512, 0), (3, 4104, 0),
+                                     (2, 32768, 8), (2, 50257, 0), (2, 65544, 0), (2, 126976, 0),
+                                     (2, 126984, 0), (2, 131072, 8), (2, 151552, 0),
+                                     (257, 151936, 0), (2, 151936, 4), (2, 155648, 0),
+                                     (2, 155656, 0)])
+def test_sample_is_softmax_then_walk(dev, dtype, N, V, pad):
+    """The one-launch draw gives the tokens of temperature_softmax followed by the walk
+    on its probabilities: around the ranges of each statistics pass, rows with padded
+    strides, greedy rows with tied maxima, -inf logits, NaN and all-masked rows, and
+    uniforms at 0 and just below 1."""
+    g = torch.Generator().manual_seed(V + N)
+    x = (torch.randn(N, V + pad, generator=g) * 2).to(dtype)
+    x[:, V // 2] = x[:, 0]
+    temps = torch.tensor([0.8, 0.0, 1.3, 0.6])[torch.arange(N) % 4].clone()
+    u = torch.rand(N, generator=g)
+    u[0] = 0.0
+    if N > 1:
+        x[1, V // 3:] = x[1, :V - V // 3].max()  # ties; first index wins
+    if N > 2:
+        x[2, : V // 2] = float("-inf")
+        u[2] = 1.0 - 2.0 ** -24
+    if N > 4:
+        x[3] = float("-inf")
+        x[4, V // 2] = float("nan")
+    if N > 8:
+        temps[5] = 0.0
+        x[5] = float("nan")
+    x, temps, u = x.to(dev)[:, :V], temps.to(dev), u.to(dev)
+    P = temperature_softmax(x, temps)
+    z = torch.zeros(N, 1, dtype=torch.int32, device=dev)
+    want = rejection_sample_tree(P.view(N, 1, V), None, z, z - 1, z.float(), u, temps == 0,
+                                 draft_mode="delta")[3]
+    got = Sampler()(x, temps, u)
+    assert got.dtype == torch.int64 and torch.equal(got, want.long())
