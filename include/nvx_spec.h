@@ -326,6 +326,45 @@ int nvx_qk_norm_rope(const void* qkv, int64_t qkv_row_stride, int32_t num_q_head
 int nvx_silu_mul(const void* gate_up, int64_t row_stride, void* out, int32_t num_rows,
                  int32_t inter, void* stream);
 
+/* ------------------------------------------------------ layers over few rows --
+ * nvx_skinny_gemm: y = x . W^T for at most 32 rows of x (bf16, fp32 accumulation), one
+ *   pass over W.  x [num_rows, in_features] with row stride x_row_stride, weight
+ *   [out_features, in_features], out [num_rows, out_features].  silu_mul != 0: weight is
+ *   [2 * out_features, in_features] (gate rows, then up rows) and
+ *   out = silu(x . gate^T) * (x . up^T).  out_features % 8 == 0, in_features % 64 == 0,
+ *   16-byte aligned rows.
+ * nvx_decoder_layer: one decoder layer (reference nanovllm/models/qwen3.py:140-160) over
+ *   at most 32 rows, its kernels enqueued by one call: add+RMSNorm, qkv projection,
+ *   nvx_qk_norm_rope with the KV store, nvx_tree_attention, o projection, add+RMSNorm,
+ *   gate/up projection with SiLU-mul, down projection.  Tensors are contiguous, with the
+ *   layouts of the entry points named.  residual may be NULL (the layer's input is then
+ *   the residual stream); residual_in_out, if not NULL, receives hidden + residual.
+ *   scratch: device memory of nvx_decoder_layer_scratch_size(args) bytes, 256-byte
+ *   aligned.  hidden_size and inter_size multiples of 64, head_dim 128.
+ */
+typedef struct nvx_decoder_layer_args {
+  const void *hidden, *residual;                        /* [num_tokens, hidden_size] */
+  void *residual_in_out, *residual_out, *out;           /* [num_tokens, hidden_size] */
+  const void *input_norm, *qkv_weight, *q_norm, *k_norm, *o_weight, *post_norm;
+  const void *gate_up_weight, *down_weight;
+  const int64_t* positions;
+  const float* cos_sin_cache;
+  void *k_cache, *v_cache;
+  const int32_t *slot_mapping, *block_tables, *cu_seqlens_q, *context_lens;
+  const uint64_t* tree_mask;
+  int64_t cache_positions;
+  int32_t num_tokens, hidden_size, inter_size, num_heads, num_kv_heads, head_dim;
+  int32_t num_seqs, max_seqlen_q, max_context_len, block_size, block_table_stride;
+  float input_eps, qk_eps, post_eps, scale;
+} nvx_decoder_layer_args;
+
+int nvx_skinny_gemm(const void* x, int64_t x_row_stride, const void* weight, void* out,
+                    int32_t num_rows, int32_t out_features, int32_t in_features,
+                    int32_t silu_mul, void* stream);
+size_t nvx_decoder_layer_scratch_size(const nvx_decoder_layer_args* args);
+int nvx_decoder_layer(const nvx_decoder_layer_args* args, void* scratch, size_t scratch_bytes,
+                      void* stream);
+
 /* ------------------------------------------------------- draft-head top-k --
  * Top-k of log_softmax(logits[r]) for every row, in one pass over the logits.
  * No counterpart in the reference (nano-vllm has no draft model); it serves the

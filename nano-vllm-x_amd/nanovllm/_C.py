@@ -17,6 +17,21 @@ DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2
 TIMER_NGRAM, TIMER_STORE_KV, TIMER_KV_COMPACT, TIMER_TREE_ATTENTION, TIMER_SOFTMAX, \
     TIMER_REJECTION, TIMER_TOPK = range(7)
 
+
+class DecoderLayerArgs(ctypes.Structure):
+    """nvx_decoder_layer_args"""
+    _fields_ = ([(n, c_void_p) for n in (
+        "hidden", "residual", "residual_in_out", "residual_out", "out", "input_norm", "qkv_weight",
+        "q_norm", "k_norm", "o_weight", "post_norm", "gate_up_weight", "down_weight", "positions",
+        "cos_sin_cache", "k_cache", "v_cache", "slot_mapping", "block_tables", "cu_seqlens_q",
+        "context_lens", "tree_mask")]
+        + [("cache_positions", c_int64)]
+        + [(n, c_int32) for n in (
+            "num_tokens", "hidden_size", "inter_size", "num_heads", "num_kv_heads", "head_dim",
+            "num_seqs", "max_seqlen_q", "max_context_len", "block_size", "block_table_stride")]
+        + [(n, c_float) for n in ("input_eps", "qk_eps", "post_eps", "scale")])
+
+
 _SIGS = {
     "nvx_version": ([], c_int32),
     "nvx_last_error": ([], ctypes.c_char_p),
@@ -51,6 +66,10 @@ _SIGS = {
                           c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p,
                           c_void_p, c_void_p, c_float, c_void_p], c_int32),
     "nvx_silu_mul": ([c_void_p, c_int64, c_void_p, c_int32, c_int32, c_void_p], c_int32),
+    "nvx_skinny_gemm": ([c_void_p, c_int64, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32,
+                         c_void_p], c_int32),
+    "nvx_decoder_layer_scratch_size": ([POINTER(DecoderLayerArgs)], c_size_t),
+    "nvx_decoder_layer": ([POINTER(DecoderLayerArgs), c_void_p, c_size_t, c_void_p], c_int32),
     "nvx_softmax_stats": ([c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_int32, c_int32,
                            c_void_p], c_int32),
     "nvx_softmax_from_stats": ([c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_int32,

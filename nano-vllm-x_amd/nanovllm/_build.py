@@ -15,7 +15,8 @@ CSRC = PKG_DIR.parent / "csrc"
 INCLUDE = PKG_DIR.parent.parent / "include"
 LIB_DIR = PKG_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libnvx_spec.so"
-SOURCES = ["capi.hip", "ngram.hip", "kvcache.hip", "sampler.hip", "attention.hip", "fused.hip", "draft.hip"]
+SOURCES = ["capi.hip", "ngram.hip", "kvcache.hip", "sampler.hip", "attention.hip", "fused.hip", "draft.hip",
+           "decode.hip"]
 ARCH = "gfx950"
 
 

@@ -4,7 +4,8 @@ Mirrors the reference's nanovllm/models/qwen3.py:14-216 (module names, fused
 qkv_proj / gate_up_proj, q/k RMSNorm, NeoX RoPE, add+RMSNorm residual stream,
 ``compute_logits`` over every row).  Tensor parallelism is left out: one process
 drives one GPU.  Dense projections are torch (hipBLASLt) GEMMs; attention,
-RMSNorm, q/k-norm + RoPE and SiLU-mul run on the HIP library.
+RMSNorm, q/k-norm + RoPE and SiLU-mul run on the HIP library.  A layer's step over a
+few rows is one library call, its projections included (layers/decoder.py).
 """
 import torch
 from torch import nn
@@ -12,6 +13,7 @@ from torch import nn
 from nanovllm import _C
 from nanovllm.layers.activation import SiluAndMul
 from nanovllm.layers.attention import Attention
+from nanovllm.layers.decoder import few_rows_layer
 from nanovllm.layers.layernorm import RMSNorm
 from nanovllm.layers.rotary_embedding import get_rope
 from nanovllm.utils.context import get_context
@@ -113,6 +115,9 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     def forward(self, positions, hidden_states, residual, aux=None):
+        few = few_rows_layer(self, Qwen3Attention, Qwen3MLP, positions, hidden_states, residual, aux)
+        if few is not None:
+            return few
         if residual is None:
             hidden_states, residual = self.input_layernorm(hidden_states), hidden_states
         else:

@@ -1,0 +1,144 @@
+"""The decoder layer's step over few rows (nvx_skinny_gemm, nvx_decoder_layer) against
+plain fp32 products and the layer's modules run one by one."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from nanovllm import _C
+from nanovllm.layers.decoder import few_rows_layer
+from nanovllm.models.qwen3 import Qwen3Attention, Qwen3DecoderLayer, Qwen3MLP, random_init_
+from nanovllm.spec.tree import ancestor_masks, random_tree
+from nanovllm.utils.context import reset_context, set_context
+from nanovllm.utils.synthetic import paged_block_tables, slots_for
+
+
+def test_validation_errors_are_reported():
+    L = _C.lib()
+    h = ctypes.c_void_p(0x100000)  # non-null host addresses: refused before any launch
+    assert L.nvx_skinny_gemm(h, 64, h, h, 33, 16, 64, 0, None) == -1
+    assert b"rows" in L.nvx_last_error()
+    assert L.nvx_skinny_gemm(h, 96, h, h, 1, 16, 96, 0, None) == -1
+    assert b"multiple" in L.nvx_last_error()
+    assert L.nvx_skinny_gemm(h, 32, h, h, 1, 16, 64, 0, None) == -1
+    assert b"row stride" in L.nvx_last_error()
+    a = _C.DecoderLayerArgs(num_tokens=1, hidden_size=64, inter_size=64, num_heads=2, num_kv_heads=1,
+                            head_dim=128, num_seqs=1, max_seqlen_q=1, max_context_len=64)
+    need = L.nvx_decoder_layer_scratch_size(ctypes.byref(a))
+    assert need > 0
+    assert L.nvx_decoder_layer(ctypes.byref(a), h, need - 1, None) == -1
+    assert b"scratch" in L.nvx_last_error()
+
+
+@pytest.mark.gpu
+# Rows at the edges of the groups of 8; columns and contraction lengths on both sides of
+# every tile width, fewer blocks than waves and uneven shares among them.
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [(8, 64), (24, 320), (3072, 192), (3080, 64), (4096, 576), (6144, 128),
+                                 (6160, 64)])
+@pytest.mark.parametrize("silu", [0, 1])
+def test_skinny_gemm(dev, rows, n, k, silu):
+    g = torch.Generator().manual_seed(rows * 7 + n + k)
+    pad = torch.randn(rows, k + 64, generator=g).to(torch.bfloat16).to(dev)  # row stride k + 64
+    x = pad[:, :k]
+    w = (torch.randn(n * (1 + silu), k, generator=g) * k ** -0.5).to(torch.bfloat16).to(dev)
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=dev)
+    _C.check(_C.lib().nvx_skinny_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), rows, n,
+                                      k, silu, _C.stream_of(x)))
+    y = x.double() @ w.double().T
+    scale = x.double().abs() @ w.double().abs().T  # bounds the fp32 sums' error
+    if silu:
+        gate, up = y.split(n, 1)
+        y = torch.nn.functional.silu(gate) * up
+        sg, su = scale.split(n, 1)
+        scale = (1.1 * sg) * up.abs() + gate.abs() * su  # |silu'| <= 1.1
+    err = (out[:rows].double() - y).abs()
+    # one rounding to bf16, k fp32 additions, expf and the division to a few ulps
+    assert (err <= y.abs() * 2.0 ** -8 + scale * (k + 16) * 2.0 ** -23).all()
+    assert (out[rows] == 7.0).all()  # nothing past the last row
+
+
+def _step(layer, hidden, residual, nodes, ctx, dev, seed):
+    """A step's context, positions and caches: `nodes` rows for each context length."""
+    rng = np.random.default_rng(seed)
+    B = len(ctx)
+    bt, nblk = paged_block_tables(np.array(ctx) + nodes, 256, rng)
+    g = torch.Generator().manual_seed(seed)
+    cache = torch.randn(2, nblk, 256, 2, 128, generator=g).to(torch.bfloat16).to(dev)
+    layer.self_attn.attn.k_cache, layer.self_attn.attn.v_cache = cache[0], cache[1]
+    masks = None
+    if nodes > 1:
+        masks = np.concatenate([ancestor_masks(random_tree(nodes, min(3, nodes - 1), rng)) for _ in ctx])
+    t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a, dtype=d)).to(dev)  # noqa: E731
+    set_context(False, cu_seqlens_q=t(np.arange(B + 1) * nodes, np.int32), max_seqlen_q=nodes,
+                slot_mapping=t(np.concatenate([slots_for(bt[b], ctx[b] + np.arange(nodes), 256)
+                                               for b in range(B)]), np.int32),
+                context_lens=t(np.array(ctx) + nodes, np.int32), block_tables=t(bt, np.int32),
+                max_context_len=max(ctx) + nodes, tree_mask=None if masks is None else t(masks, np.int64))
+    return t(np.concatenate([c + np.arange(nodes) for c in ctx]), np.int64), cache
+
+
+def _layer(dev):
+    from transformers import Qwen3Config
+    cfg = Qwen3Config(hidden_size=512, intermediate_size=1536, num_hidden_layers=1,
+                      num_attention_heads=4, num_key_value_heads=2, head_dim=128, vocab_size=512,
+                      max_position_embeddings=4096, rope_theta=1000000, rms_norm_eps=1e-6,
+                      hidden_act="silu", attention_bias=False)
+    torch.set_default_dtype(torch.bfloat16)  # the rotary table stays fp32
+    try:
+        layer = Qwen3DecoderLayer(cfg)
+    finally:
+        torch.set_default_dtype(torch.float32)
+    return random_init_(layer.to(dev), std=0.05)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ctx,nodes", [([300], 1), ([5, 700, 90], 1), ([40, 0, 513, 64], 5),
+                                       ([130] * 32, 1)])
+@pytest.mark.parametrize("first", [False, True])
+def test_layer_matches_its_modules(dev, ctx, nodes, first):
+    layer, N = _layer(dev), len(ctx) * nodes
+    g = torch.Generator().manual_seed(N)
+    hidden = torch.randn(N, 512, generator=g).to(torch.bfloat16).to(dev)
+    residual = None if first else torch.randn(N, 512, generator=g).to(torch.bfloat16).to(dev)
+    got, aux = [], [[], []]
+    try:
+        for i in (0, 1):
+            positions, cache = _step(layer, hidden, residual, nodes, ctx, dev, 3)
+            with torch.set_grad_enabled(i == 1):  # gradients: module by module
+                used = few_rows_layer(layer, Qwen3Attention, Qwen3MLP, positions, hidden, residual)
+                assert (used is None) == (i == 1)
+                got.append((*layer(positions, hidden, residual, aux[i]), cache))
+    finally:
+        reset_context()
+    assert torch.equal(aux[0][0], aux[1][0])
+    # a dozen roundings to bf16 (2^-9 each) meet in the outputs, the projections' sums being
+    # the only difference: a few per mille
+    for a, b in zip(*got):
+        a, b = a.detach().double(), b.detach().double()
+        assert ((a - b).norm() / b.norm()) < 1e-2
+
+
+@pytest.mark.gpu
+def test_modules_run_where_something_watches_or_replaces_them(dev):
+    layer = _layer(dev)
+    hidden = torch.randn(2, 512).to(torch.bfloat16).to(dev)
+    try:
+        with torch.no_grad():
+            positions, _ = _step(layer, hidden, None, 1, [30, 50], dev, 1)
+            call = lambda h=hidden: few_rows_layer(layer, Qwen3Attention, Qwen3MLP, positions, h, None)  # noqa: E731
+            assert call() is not None
+            seen = []
+            hook = layer.mlp.down_proj.register_forward_hook(lambda *a: seen.append(1))
+            assert call() is None
+            layer(positions, hidden, None)
+            assert seen
+            hook.remove()
+            assert call() is not None
+            assert call(hidden.float()) is None
+            assert call(torch.randn(33, 512, device=dev).to(torch.bfloat16)) is None
+            layer.self_attn.o_proj = torch.nn.Sequential(layer.self_attn.o_proj)
+            assert call() is None
+    finally:
+        reset_context()
