@@ -381,6 +381,11 @@ int nvx_topk_logprobs(const void* logits, int32_t logits_dtype, int64_t logits_r
                       int32_t num_rows, int32_t vocab, int32_t k, int32_t* out_tokens,
                       float* out_logprobs, void* stream);
 
+/* nvx_topk_logprobs_i64: the same with int64 token ids. */
+int nvx_topk_logprobs_i64(const void* logits, int32_t logits_dtype, int64_t logits_row_stride,
+                          int32_t num_rows, int32_t vocab, int32_t k, int64_t* out_tokens,
+                          float* out_logprobs, void* stream);
+
 /* ------------------------------------------------------------------ timing --
  * Optional per-entry-point HIP-event timing on the launch stream (used by the
  * benchmark to measure kernel durations in its timed region).

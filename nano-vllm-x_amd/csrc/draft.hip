@@ -10,13 +10,15 @@
 //    j-th largest 64-bit key  (order-preserving bits of the value) << 32 | ~index,
 //    so a larger key ranks first and equal values rank by the lower token id.
 //    A value can only enter when it is >= a threshold: the list's k-th value, and
-//    from the start the k-th largest of the wave's first-vector lane maxima (k
-//    distinct elements, so a lower bound of the row's k-th largest value).  After
-//    the first vectors candidates are rare; each is inserted with one lane shift.
+//    from the start a lower bound of the row's k-th largest value that the workgroup
+//    takes from its first loads.  Candidates are rare; each is inserted with one lane
+//    shift.
 //  * the waves' lists meet in LDS, where each key's rank among them (the number
 //    of larger keys) is its output slot.
 // Rows must be free of NaN.  Outputs per row are ordered by descending
 // log-probability, ties to the lower token id.
+#include <type_traits>
+
 #include "nvx_internal.h"
 
 namespace {
@@ -90,10 +92,18 @@ struct WaveTopK {
   }
 };
 
-template <typename VT, int NT>
+// Bound by each wave's work between its loads: 256 rows of 32,000 bf16 logits are one
+// workgroup per CU and 64 KB per row.  The first chunk (kUnroll vectors per thread) sets
+// the threshold for the whole workgroup -- the largest over its waves of the k-th largest
+// lane maximum, each a lower bound of the row's k-th largest value -- so of a row's
+// values a few dozen, not a few dozen per wave, are offered to the lists; and every chunk
+// is kUnroll guarded loads in flight, the last one too.
+// [256, 32000] bf16, k = 8: 11.8 us; a threshold per wave and a tail of single loads
+// took 16.0 us.
+template <typename VT, int NT, typename TokT>
 __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict__ logits,
                                                            int64_t stride, int V, int k,
-                                                           int32_t* __restrict__ out_tok,
+                                                           TokT* __restrict__ out_tok,
                                                            float* __restrict__ out_lp) {
   using Tr = nvx::VecTraits<VT>;
   constexpr int P = Tr::kPer;
@@ -108,34 +118,28 @@ __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict_
   WaveTopK tk;
   tk.k = k;
   tk.lane = lane;
-  {
-    float lm = -INFINITY;
-    if (tid < nvec) {
-      float x[P];
-      Tr::expand(src[tid], x);
-#pragma unroll
-      for (int e = 0; e < P; ++e) lm = fmaxf(lm, x[e]);
-    }
-    tk.thr0 = wave_kth_largest(lm, k, lane);
-    tk.thr = tk.thr0;
-  }
+  tk.thr0 = tk.thr = -INFINITY;
 
-  // Lane l of wave w reads vectors w*64 + l + t*NT, t = 0, 1, ...; the loops run on
-  // the wave's first vector j so that every lane takes every iteration.
+  // Lane l of wave w reads vectors w*64 + l + t*NT, t = 0, 1, ...; the loop runs on the
+  // workgroup's first vector j so that every lane takes every iteration.
   float m = -INFINITY, m2 = -INFINITY, s = 0.f;
-  int j = wid * nvx::kWave;
-  for (; j + (nvx::kWave - 1) + (kUnroll - 1) * NT < nvec; j += kUnroll * NT) {
-    const int i = j + lane;
+  auto chunk = [&](int j, auto whole) {
+    constexpr bool kWhole = decltype(whole)::value;  // every thread's vectors are in the row
+    const int i = j + tid;
     uint4 w[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) w[u] = nvx::ld_stream(src + i + u * NT);
+    for (int u = 0; u < kUnroll; ++u)
+      w[u] = nvx::ld_stream(src + (kWhole ? i + u * NT : min(i + u * NT, nvec - 1)));
     float x[kUnroll][P];
     float lm = -INFINITY;
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       Tr::expand(w[u], x[u]);
 #pragma unroll
-      for (int e = 0; e < P; ++e) lm = fmaxf(lm, x[u][e]);
+      for (int e = 0; e < P; ++e) {
+        if (!kWhole) x[u][e] = i + u * NT < nvec ? x[u][e] : -INFINITY;
+        lm = fmaxf(lm, x[u][e]);
+      }
     }
     if (lm > m) {
       const float m2n = lm * kLog2e;
@@ -154,41 +158,21 @@ __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict_
         }
       s += a0 + a1;
     }
+    if (j == 0) {
+      tk.thr0 = nvx::block_max<NT>(wave_kth_largest(lm, k, lane), red);
+      tk.thr = tk.thr0;
+    }
     if (__ballot(lm >= tk.thr)) {
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u)
 #pragma unroll
-        for (int e = 0; e < P; ++e) tk.offer(x[u][e], (i + u * NT) * P + e);
+        for (int e = 0; e < P; ++e)
+          tk.offer(x[u][e], (i + u * NT) * P + e, kWhole || i + u * NT < nvec);
     }
-  }
-  for (; j < nvec; j += NT) {  // the rest, one vector per lane per iteration
-    const int i = j + lane;
-    const bool ok = i < nvec;
-    float x[P];
-    float lm = -INFINITY;
-    if (ok) {
-      Tr::expand(src[i], x);
-#pragma unroll
-      for (int e = 0; e < P; ++e) lm = fmaxf(lm, x[e]);
-      if (lm > m) {
-        const float m2n = lm * kLog2e;
-        s = (m == -INFINITY) ? 0.f : s * __builtin_amdgcn_exp2f(m2 - m2n);
-        m = lm;
-        m2 = m2n;
-      }
-      if (m != -INFINITY) {
-#pragma unroll
-        for (int e = 0; e < P; ++e) s += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], kLog2e, -m2));
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < P; ++e) x[e] = -INFINITY;
-    }
-    if (__ballot(ok && lm >= tk.thr)) {
-#pragma unroll
-      for (int e = 0; e < P; ++e) tk.offer(x[e], i * P + e, ok);
-    }
-  }
+  };
+  int j = 0;
+  for (; j + kUnroll * NT <= nvec; j += kUnroll * NT) chunk(j, std::true_type{});
+  if (j < nvec) chunk(j, std::false_type{});
 
   const float M = nvx::block_max<NT>(m, red);
   const float part = (m == -INFINITY) ? 0.f : s * __builtin_amdgcn_exp2f(m2 - M * kLog2e);
@@ -203,32 +187,31 @@ __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict_
       int rank = 0;
       for (int u = 0; u < NW * k; ++u) rank += lists[u] > c ? 1 : 0;
       if (rank < k) {
-        out_tok[(int64_t)row * k + rank] = (int32_t)~(uint32_t)c;
+        out_tok[(int64_t)row * k + rank] = (TokT)(int32_t)~(uint32_t)c;
         out_lp[(int64_t)row * k + rank] = (from_ord((uint32_t)(c >> 32)) - M) - lnS;
       }
     }
   }
 }
 
-template <typename VT>
-void launch(const void* logits, int64_t stride, int rows, int V, int k, int32_t* tok, float* lp,
+template <typename VT, typename TokT>
+void launch(const void* logits, int64_t stride, int rows, int V, int k, TokT* tok, float* lp,
             hipStream_t s) {
   const VT* x = reinterpret_cast<const VT*>(logits);
   // Few rows: wide workgroups keep enough loads in flight per CU; many rows:
   // narrow ones keep the per-wave lists short relative to the row.
   if (rows >= 1024)
-    hipLaunchKernelGGL((topk_logprobs_kernel<VT, 256>), dim3(rows), dim3(256), 0, s, x, stride, V,
-                       k, tok, lp);
+    hipLaunchKernelGGL((topk_logprobs_kernel<VT, 256, TokT>), dim3(rows), dim3(256), 0, s, x, stride,
+                       V, k, tok, lp);
   else
-    hipLaunchKernelGGL((topk_logprobs_kernel<VT, 1024>), dim3(rows), dim3(1024), 0, s, x, stride,
+    hipLaunchKernelGGL((topk_logprobs_kernel<VT, 1024, TokT>), dim3(rows), dim3(1024), 0, s, x, stride,
                        V, k, tok, lp);
 }
 
-}  // namespace
-
-extern "C" int nvx_topk_logprobs(const void* logits, int32_t logits_dtype, int64_t logits_row_stride,
-                                 int32_t num_rows, int32_t vocab, int32_t k, int32_t* out_tokens,
-                                 float* out_logprobs, void* stream) {
+template <typename TokT>
+int topk_logprobs_run(const void* logits, int32_t logits_dtype, int64_t logits_row_stride,
+                      int32_t num_rows, int32_t vocab, int32_t k, TokT* out_tokens,
+                      float* out_logprobs, void* stream) {
   nvx::clear_error();
   NVX_CHECK(logits_dtype == NVX_DTYPE_BF16 || logits_dtype == NVX_DTYPE_F32,
             "topk_logprobs: logits must be bf16 or fp32 (dtype code %d)", logits_dtype);
@@ -246,9 +229,26 @@ extern "C" int nvx_topk_logprobs(const void* logits, int32_t logits_dtype, int64
   hipStream_t s = (hipStream_t)stream;
   nvx::TimerScope timer(NVX_TIMER_TOPK, s);
   if (logits_dtype == NVX_DTYPE_BF16)
-    launch<uint16_t>(logits, logits_row_stride, num_rows, vocab, k, out_tokens, out_logprobs, s);
+    launch<uint16_t, TokT>(logits, logits_row_stride, num_rows, vocab, k, out_tokens, out_logprobs, s);
   else
-    launch<float>(logits, logits_row_stride, num_rows, vocab, k, out_tokens, out_logprobs, s);
+    launch<float, TokT>(logits, logits_row_stride, num_rows, vocab, k, out_tokens, out_logprobs, s);
   NVX_LAUNCHED();
   return NVX_OK;
+}
+
+}  // namespace
+
+extern "C" int nvx_topk_logprobs(const void* logits, int32_t logits_dtype, int64_t logits_row_stride,
+                                 int32_t num_rows, int32_t vocab, int32_t k, int32_t* out_tokens,
+                                 float* out_logprobs, void* stream) {
+  return topk_logprobs_run(logits, logits_dtype, logits_row_stride, num_rows, vocab, k, out_tokens,
+                           out_logprobs, stream);
+}
+
+extern "C" int nvx_topk_logprobs_i64(const void* logits, int32_t logits_dtype,
+                                     int64_t logits_row_stride, int32_t num_rows, int32_t vocab,
+                                     int32_t k, int64_t* out_tokens, float* out_logprobs,
+                                     void* stream) {
+  return topk_logprobs_run(logits, logits_dtype, logits_row_stride, num_rows, vocab, k, out_tokens,
+                           out_logprobs, stream);
 }

@@ -86,6 +86,8 @@ _SIGS = {
                                                c_void_p, c_void_p, c_size_t, c_void_p], c_int32),
     "nvx_topk_logprobs": ([c_void_p, c_int32, c_int64, c_int32, c_int32, c_int32, c_void_p,
                            c_void_p, c_void_p], c_int32),
+    "nvx_topk_logprobs_i64": ([c_void_p, c_int32, c_int64, c_int32, c_int32, c_int32, c_void_p,
+                               c_void_p, c_void_p], c_int32),
     "nvx_rejection_walk_max_width": ([c_int32], c_int32),
     "nvx_timing_enable": ([c_int32], c_int32),
     "nvx_timing_read": ([c_int32, POINTER(c_double), POINTER(c_int64)], c_int32),

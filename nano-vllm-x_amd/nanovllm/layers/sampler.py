@@ -48,13 +48,13 @@ def topk_logprobs(logits: torch.Tensor, k: int):
     if logits.dtype not in _DTYPE_CODE:
         raise ValueError(f"topk_logprobs: unsupported logits dtype {logits.dtype}")
     N, V = logits.shape
-    tok = torch.empty(N, k, dtype=torch.int32, device=logits.device)
+    tok = torch.empty(N, k, dtype=torch.int64, device=logits.device)
     lp = torch.empty(N, k, dtype=torch.float32, device=logits.device)
     _C.require_cuda(logits)
-    _C.check(_C.lib().nvx_topk_logprobs(
+    _C.check(_C.lib().nvx_topk_logprobs_i64(
         _C.ptr(logits), _DTYPE_CODE[logits.dtype], logits.stride(0), N, V, k, _C.ptr(tok),
         _C.ptr(lp), _C.stream_of(logits)))
-    return lp, tok.long()
+    return lp, tok
 
 
 def _i32(t):

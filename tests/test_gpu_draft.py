@@ -79,3 +79,19 @@ def test_k_equals_vocab_and_monotone_rows(dev):
 def test_empty_batch(dev):
     lp, tok = topk_logprobs(torch.zeros(0, 512, device=dev), 4)
     assert lp.shape == (0, 4) and tok.shape == (0, 4)
+
+
+@pytest.mark.gpu
+# One value on both sides of the first chunk of loads (4 vectors of every thread: 32,768
+# bf16 or 16,384 fp32 values at 1024 threads, a quarter at 1024 rows and more), the
+# largest values in its last vector, in the last one of the row, or equal throughout.
+@pytest.mark.parametrize("rows,V", [(3, 32760), (3, 32768), (3, 32776), (3, 65544), (1024, 8184),
+                                    (1024, 8200), (2, 8), (2, 520)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_chunk_edges(dev, rows, V, dtype):
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(rows, V, generator=g)
+    x[0, -8:] += 20.0
+    x[1, max(0, min(V, 32768) - 8):min(V, 32768)] += 20.0
+    x[-1] = 1.5
+    check(dev, x.to(dtype), 8)
