@@ -210,6 +210,23 @@ int nvx_rejection_sample_tree(const float* target_probs, int64_t p_seq_stride,
                               int32_t* next_token, void* workspace, size_t workspace_bytes,
                               void* stream);
 
+/* nvx_rejection_sample_chain: nvx_rejection_sample_tree (draft_mode 0) on the chain of
+ * num_draft draft tokens of each sequence (Leviathan et al. 2023, Alg. 1), with the
+ * chain's inputs and outputs as a caller holds them: one launch.
+ *   target_probs fp32 [num_seqs, num_draft + 1, vocab]  draft_probs fp32 [num_seqs, >= num_draft, vocab]
+ *   draft_tokens int32 or int64 [num_seqs, num_draft]   uniforms fp32 [num_seqs, num_draft]
+ *   accepted_len, recovered (-1 when all were accepted), bonus (-1 otherwise) int32 [num_seqs]
+ *   out_tokens   int32 [num_seqs, num_draft + 1] (-1 padded)
+ * Other arguments as nvx_rejection_sample_tree.
+ */
+int nvx_rejection_sample_chain(const float* target_probs, int64_t p_seq_stride,
+                               const float* draft_probs, int64_t q_seq_stride, int32_t vocab,
+                               const void* draft_tokens, int32_t tokens_are_i64, int32_t num_draft,
+                               const float* uniforms, const float* final_uniforms,
+                               const uint8_t* greedy, int32_t num_seqs, int32_t* accepted_len,
+                               int32_t* recovered, int32_t* bonus, int32_t* out_tokens,
+                               void* workspace, size_t workspace_bytes, void* stream);
+
 /* nvx_rejection_walk_workspace_size: no counterpart in the reference.  Bytes of the
  * exchange workspace a tree / chain rejection walk of num_seqs sequences needs
  * (1,280 per sequence; 0 for num_seqs <= 0).  Sequence b always uses the same
@@ -290,6 +307,19 @@ int nvx_rejection_sample_tree_logits_lazy(const void* logits, int32_t logits_dty
                                           int32_t num_seqs, int32_t* path, int32_t* accepted_len,
                                           int32_t* out_tokens, int32_t* next_token,
                                           void* workspace, size_t workspace_bytes, void* stream);
+
+/* nvx_rejection_verify_logits: nvx_rejection_sample_tree_logits_lazy with one temperature
+ * per sequence (temperatures fp32 [num_seqs]); sequences of temperature 0 are greedy.
+ */
+int nvx_rejection_verify_logits(const void* logits, int32_t logits_dtype, int64_t logits_row_stride,
+                                const float* temperatures, float* stats_out,
+                                const float* draft_probs, int64_t q_seq_stride, int32_t vocab,
+                                const int32_t* tokens, const int32_t* parents,
+                                const int32_t* num_nodes, int32_t node_stride,
+                                const float* uniforms, const float* final_uniforms,
+                                int32_t draft_mode, int32_t num_seqs, int32_t* path,
+                                int32_t* accepted_len, int32_t* out_tokens, int32_t* next_token,
+                                void* workspace, size_t workspace_bytes, void* stream);
 
 /* -------------------------------------------------- fused model layers --
  * Elementwise layers of the target model around the verify-path attention, each

@@ -59,6 +59,10 @@ _SIGS = {
                                    c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
                                    c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
                                    c_void_p, c_size_t, c_void_p], c_int32),
+    "nvx_rejection_sample_chain": ([c_void_p, c_int64, c_void_p, c_int64, c_int32, c_void_p, c_int32,
+                                    c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
+                                    c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
+                                   c_int32),
     "nvx_rejection_walk_workspace_size": ([c_int32], c_size_t),
     "nvx_rmsnorm": ([c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32,
                      c_float, c_void_p], c_int32),
@@ -84,6 +88,10 @@ _SIGS = {
                                                c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
                                                c_int32, c_int32, c_void_p, c_void_p, c_void_p,
                                                c_void_p, c_void_p, c_size_t, c_void_p], c_int32),
+    "nvx_rejection_verify_logits": ([c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_int64,
+                                     c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
+                                     c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p,
+                                     c_void_p, c_void_p, c_size_t, c_void_p], c_int32),
     "nvx_topk_logprobs": ([c_void_p, c_int32, c_int64, c_int32, c_int32, c_int32, c_void_p,
                            c_void_p, c_void_p], c_int32),
     "nvx_topk_logprobs_i64": ([c_void_p, c_int32, c_int64, c_int32, c_int32, c_int32, c_void_p,

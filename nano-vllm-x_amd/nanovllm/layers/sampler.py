@@ -61,6 +61,13 @@ def _i32(t):
     return t.to(torch.int32).contiguous()
 
 
+def _flags(t, dev):
+    """bool (or 0/1) flags as uint8, without a copy where they are bool already."""
+    if t.dtype is torch.bool and t.device == dev and t.is_contiguous():
+        return t.view(torch.uint8)
+    return t.to(device=dev, dtype=torch.uint8).contiguous()
+
+
 _WALK_WS = {}  # (device index, stream) -> zero-filled uint8 tensor, grown on demand
 
 
@@ -118,7 +125,7 @@ def rejection_sample_tree(target_probs, draft_probs, tokens, parents, uniforms, 
     tokens, parents = _i32(tokens), _i32(parents)
     uniforms = uniforms.to(torch.float32).contiguous()
     final_uniforms = final_uniforms.to(torch.float32).contiguous()
-    g = None if greedy is None else greedy.to(device=dev, dtype=torch.uint8).contiguous()
+    g = None if greedy is None else _flags(greedy, dev)
     nn_ = None if num_nodes is None else _i32(num_nodes)
     path = torch.empty(B, T, dtype=torch.int32, device=dev)
     acc = torch.empty(B, dtype=torch.int32, device=dev)
@@ -212,7 +219,7 @@ def rejection_sample_tree_logits(logits, temperatures, stats, draft_probs, token
     tokens, parents = _i32(tokens), _i32(parents)
     uniforms = uniforms.to(torch.float32).contiguous()
     final_uniforms = final_uniforms.to(torch.float32).contiguous()
-    g = None if greedy is None else greedy.to(device=dev, dtype=torch.uint8).contiguous()
+    g = None if greedy is None else _flags(greedy, dev)
     nn_ = None if num_nodes is None else _i32(num_nodes)
     path = torch.empty(B, T, dtype=torch.int32, device=dev)
     acc = torch.empty(B, dtype=torch.int32, device=dev)
@@ -241,6 +248,14 @@ def rejection_sample_tree_logits_lazy(logits, temperatures, draft_probs, tokens,
     rejection_sample_tree(softmax_from_stats(logits, temperatures, stats)) for any stats
     that hold stats_out's values on the visited rows.  Returns (path, accepted_len,
     out_tokens, next_token, stats_out)."""
+    return _walk_logits_lazy(logits, temperatures, draft_probs, tokens, parents, uniforms,
+                             final_uniforms, greedy, num_nodes, draft_mode, workspace, stats_out)
+
+
+def _walk_logits_lazy(logits, temperatures, draft_probs, tokens, parents, uniforms, final_uniforms,
+                      greedy, num_nodes, draft_mode, workspace, stats_out, per_seq=False):
+    """rejection_sample_tree_logits_lazy; per_seq: temperatures [B], and the sequences of
+    temperature 0 are the greedy ones (greedy is not given)."""
     B, T = tokens.shape
     if not stats_eligible(logits) or logits.shape[0] != B * T:
         raise ValueError("rejection_sample_tree_logits_lazy: logits must be [B*T, V] "
@@ -256,8 +271,9 @@ def rejection_sample_tree_logits_lazy(logits, temperatures, draft_probs, tokens,
         raise ValueError("rejection_sample_tree_logits_lazy: at most 64 nodes per tree")
     dev = logits.device
     temperatures = temperatures.to(device=dev, dtype=torch.float32).contiguous()
-    if temperatures.numel() != B * T:
-        raise ValueError("rejection_sample_tree_logits_lazy: one temperature per logits row")
+    if temperatures.numel() != (B if per_seq else B * T):
+        raise ValueError("rejection_sample_tree_logits_lazy: one temperature per "
+                         + ("sequence" if per_seq else "logits row"))
     if stats_out is not None and (stats_out.shape != (B * T, 2) or stats_out.dtype != torch.float32
                                   or not stats_out.is_contiguous()):
         raise ValueError("rejection_sample_tree_logits_lazy: stats_out must be contiguous fp32 "
@@ -265,7 +281,7 @@ def rejection_sample_tree_logits_lazy(logits, temperatures, draft_probs, tokens,
     tokens, parents = _i32(tokens), _i32(parents)
     uniforms = uniforms.to(torch.float32).contiguous()
     final_uniforms = final_uniforms.to(torch.float32).contiguous()
-    g = None if greedy is None else greedy.to(device=dev, dtype=torch.uint8).contiguous()
+    g = None if greedy is None else _flags(greedy, dev)
     nn_ = None if num_nodes is None else _i32(num_nodes)
     path = torch.empty(B, T, dtype=torch.int32, device=dev)
     acc = torch.empty(B, dtype=torch.int32, device=dev)
@@ -274,12 +290,16 @@ def rejection_sample_tree_logits_lazy(logits, temperatures, draft_probs, tokens,
     _C.require_cuda(logits, temperatures, draft_probs, tokens, parents, uniforms, final_uniforms,
                     g, nn_, workspace, stats_out)
     ws, ws_bytes = walk_workspace(B, dev, workspace)
-    _C.check(_C.lib().nvx_rejection_sample_tree_logits_lazy(
-        _C.ptr(logits), _DTYPE_CODE[logits.dtype], logits.stride(0), _C.ptr(temperatures),
-        _C.ptr(stats_out), None if delta else _C.ptr(draft_probs),
-        0 if delta else draft_probs.stride(0), V, _C.ptr(tokens), _C.ptr(parents), _C.ptr(nn_), T,
-        _C.ptr(uniforms), _C.ptr(final_uniforms), _C.ptr(g), 1 if delta else 0, B, _C.ptr(path),
-        _C.ptr(acc), _C.ptr(out_tokens), _C.ptr(nxt), _C.ptr(ws), ws_bytes, _C.stream_of(logits)))
+    head = (_C.ptr(logits), _DTYPE_CODE[logits.dtype], logits.stride(0), _C.ptr(temperatures),
+            _C.ptr(stats_out), None if delta else _C.ptr(draft_probs),
+            0 if delta else draft_probs.stride(0), V, _C.ptr(tokens), _C.ptr(parents), _C.ptr(nn_), T,
+            _C.ptr(uniforms), _C.ptr(final_uniforms))
+    tail = (1 if delta else 0, B, _C.ptr(path), _C.ptr(acc), _C.ptr(out_tokens), _C.ptr(nxt),
+            _C.ptr(ws), ws_bytes, _C.stream_of(logits))
+    if per_seq:
+        _C.check(_C.lib().nvx_rejection_verify_logits(*head, *tail))
+    else:
+        _C.check(_C.lib().nvx_rejection_sample_tree_logits_lazy(*head, _C.ptr(g), *tail))
     return path, acc, out_tokens, nxt, stats_out
 
 
@@ -294,18 +314,34 @@ def rejection_sample_chain(target_probs, draft_probs, draft_token_ids, uniforms,
     """
     B, k1, V = target_probs.shape
     k = k1 - 1
+    if target_probs.dtype != torch.float32 or target_probs.stride(2) != 1 \
+            or target_probs.stride(1) != V:
+        raise ValueError("rejection_sample_chain: target_probs must be fp32 with contiguous rows")
+    if draft_probs is None or draft_probs.dtype != torch.float32 or draft_probs.stride(2) != 1 \
+            or draft_probs.stride(1) != V or draft_probs.shape[2] != V:
+        raise ValueError("rejection_sample_chain: draft_probs must be fp32 [B, k, V] with "
+                         "contiguous rows")
+    if k1 > 64:
+        raise ValueError("rejection_sample_chain: at most 63 draft tokens")
     dev = target_probs.device
-    tok = torch.zeros(B, k1, dtype=torch.int32, device=dev)
-    tok[:, 1:] = draft_token_ids.to(torch.int32)
-    u = torch.zeros(B, k1, dtype=torch.float32, device=dev)
-    u[:, 1:] = uniforms
-    parents = (torch.arange(k1, dtype=torch.int32, device=dev) - 1).expand(B, k1).contiguous()
-    _, acc, toks, nxt = rejection_sample_tree(target_probs, draft_probs, tok, parents, u,
-                                              final_uniforms, greedy)
-    full = acc == k
-    recovered = torch.where(full, torch.full_like(nxt, -1), nxt)
-    bonus = torch.where(full, nxt, torch.full_like(nxt, -1))
-    return acc, recovered, bonus, toks
+    tok = draft_token_ids
+    if tok.dtype not in (torch.int32, torch.int64):
+        tok = tok.to(torch.int32)
+    tok = tok.to(dev).expand(B, k).contiguous()
+    u = uniforms.to(device=dev, dtype=torch.float32).expand(B, k).contiguous()
+    final_uniforms = final_uniforms.to(torch.float32).contiguous()
+    g = None if greedy is None else _flags(greedy, dev)
+    # accepted_len, recovered, bonus [B] and tokens [B, k + 1] in one allocation
+    out = torch.empty(B * (k + 4), dtype=torch.int32, device=dev)
+    acc, recovered, bonus, toks = out.split([B, B, B, B * k1])
+    _C.require_cuda(target_probs, draft_probs, final_uniforms)
+    ws, ws_bytes = walk_workspace(B, dev)
+    _C.check(_C.lib().nvx_rejection_sample_chain(
+        _C.ptr(target_probs), target_probs.stride(0), _C.ptr(draft_probs), draft_probs.stride(0), V,
+        _C.ptr(tok), tok.dtype is torch.int64, k, _C.ptr(u), _C.ptr(final_uniforms), _C.ptr(g), B,
+        _C.ptr(acc), _C.ptr(recovered), _C.ptr(bonus), _C.ptr(toks), _C.ptr(ws), ws_bytes,
+        _C.stream_of(target_probs)))
+    return acc, recovered, bonus, toks.view(B, k1)
 
 
 class Sampler(nn.Module):
@@ -355,12 +391,12 @@ class RejectionSampler(nn.Module):
         V = target_logits.shape[-1]
         temps = temperatures.to(device=target_logits.device, dtype=torch.float32)
         rows = target_logits.view(B * T, V)
-        row_temps = temps.repeat_interleave(T)
         mode = "delta" if draft_probs is None else "stochastic"
         if stats_eligible(rows) and self.lazy:
-            return rejection_sample_tree_logits_lazy(rows, row_temps, draft_probs, tokens, parents,
-                                                     uniforms, final_uniforms, temps == 0,
-                                                     num_nodes, mode, stats_out=stats_out)[:4]
+            return _walk_logits_lazy(rows, temps, draft_probs, tokens, parents, uniforms,
+                                     final_uniforms, None, num_nodes, mode, None, stats_out,
+                                     per_seq=True)[:4]
+        row_temps = temps.repeat_interleave(T)
         if stats_eligible(rows):
             # fused: one statistics pass over the logits, then the walk recomputes the
             # probabilities of the rows it visits (no fp32 probability rows written)

@@ -525,3 +525,31 @@ def test_sample_is_softmax_then_walk(dev, dtype, N, V, pad):
                                  draft_mode="delta")[3]
     got = Sampler()(x, temps, u)
     assert got.dtype == torch.int64 and torch.equal(got, want.long())
+
+
+@pytest.mark.gpu
+# The shortest and longest chains, odd and even vocabularies, one to many workgroups per
+# sequence; draft tokens as int64, int32, a strided view and (as before) other integers,
+# flags as bool and as bytes.
+@pytest.mark.parametrize("B,k,V,tok_dtype,greedy", [
+    (1, 1, 1003, torch.int64, None), (9, 4, 50257, torch.int64, torch.bool),
+    (70, 3, 2048, torch.int32, torch.uint8), (3, 63, 512, torch.int64, None),
+    (5, 2, 32000, torch.int16, torch.bool)])
+def test_chain_forms(dev, B, k, V, tok_dtype, greedy):
+    g = torch.Generator().manual_seed(B * 100 + k)
+    tl = torch.randn(B, k + 1, V, generator=g) * 2
+    P = torch.softmax(tl, -1).to(dev)
+    Q = torch.softmax(tl[:, :k] + 0.5 * torch.randn(B, k, V, generator=g), -1)
+    draft = torch.multinomial(Q.view(B * k, V), 1, generator=g).view(B, k)
+    U, Uf = torch.rand(B, k, generator=g), torch.rand(B, generator=g)
+    flags = None if greedy is None else torch.arange(B) % 3 == 0
+    wide = torch.zeros(B, 2 * k, dtype=tok_dtype, device=dev)
+    wide[:, ::2] = draft.to(dev, tok_dtype)
+    ref = osamp.rejection_sample_chain(P.cpu().numpy(), Q.numpy(), draft.numpy().astype(np.int32),
+                                       U.numpy(), Uf.numpy(),
+                                       np.zeros(B, bool) if flags is None else flags.numpy())
+    for tok in (draft.to(dev, tok_dtype), wide[:, ::2]):
+        out = rejection_sample_chain(P, Q.to(dev), tok, U.to(dev), Uf.to(dev),
+                                     None if flags is None else flags.to(dev, greedy))
+        for a, r in zip(out, ref):
+            assert a.dtype == torch.int32 and np.array_equal(a.cpu().numpy(), r)
