@@ -169,28 +169,12 @@ void tree_attn_kernel(AttnParams p) {
   const int head = hk * p.G + (row_ok ? r % p.G : 0);
   const int token = q0 + node;
 
-  // Q^T fragments (B operand of S^T = K.Q^T): d = 16*s + 8*g + [0..7].
-  bf16x8 bq[8];
-  {
-    const bool ld = row_ok && token < p.total_q;
-    const uint16_t* qrow = p.q + ((int64_t)token * p.Hq + head) * kD + 8 * g;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (ld) v = *reinterpret_cast<const uint4*>(qrow + 16 * s);
-      bf16x8 x = __builtin_bit_cast(bf16x8, v);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = (__bf16)((float)x[e] * p.scale_log2);
-      bq[s] = x;
-    }
-  }
   const bool use_tree = p.tree_mask != nullptr;
   // First key that some row of this wave cannot see: the tree start with a tree mask;
   // causal, one past the key of the wave's first node (every row of the wave sees the
   // keys before it).  Chunks wholly before it need no mask -- in causal prefill
   // (base 0) only the chunks on the diagonal of the wave's rows do.
   const int mask_from = use_tree ? base : base + (row0 + wave * 32) / p.G + 1;
-  const uint64_t mbits = (use_tree && row_ok && token < p.total_q) ? p.tree_mask[token] : 0ull;
 
   // Keys beyond the last node of this chunk's rows are masked for every row.
   const int last_node = min(qlen - 1, (row0 + W * 32 - 1) / p.G);
@@ -206,19 +190,8 @@ void tree_attn_kernel(AttnParams p) {
   const int bs = p.block_size;
   const uint32_t ring_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring;
 
-  // This split's block-table entries go to LDS once, so the loop reads page ids
-  // without touching the vector-memory counter the DMA pipeline waits on.
   const int page0 = (c0 * kKC) / bs;
   const int npages = c1 > c0 ? ((c1 * kKC - 1) / bs - page0 + 1) : 0;
-  for (int i = tid; i < npages; i += W * 64)
-    pages[i] = (page0 + i < p.bt_stride) ? bt[page0 + i] : -1;
-  // Make every prologue global load (Q, mask, pages) complete here, before the
-  // first LDS-DMA is queued behind them.
-#pragma unroll
-  for (int s = 0; s < 8; ++s) asm volatile("" : : "v"(bq[s]));
-  asm volatile("" : : "v"(mbits));
-  __syncthreads();
-
   // The PER LDS-DMA loads of this wave for one chunk: load j of wave w fills 4 rows
   // (1 KB) of the K (first 16 loads) or V (last 16) tile; lane i fetches row
   // 4*(ii%16) + i/16, logical segment (i%16)^swz(row), so the tile lands swizzled.
@@ -241,10 +214,9 @@ void tree_attn_kernel(AttnParams p) {
   // The chunk to issue next, as (page index in the LDS table, key offset in the page),
   // advanced by one chunk per issue (no division in the loop).
   int is_page = 0, is_off = (c0 * kKC) % bs;
-  auto issue_chunk = [&](int c, auto stage) {
+  auto issue_chunk_of = [&](int c, int32_t blk, auto stage) {
     constexpr int ST = decltype(stage)::value;
     const int pos0 = c * kKC;
-    const int32_t blk = __builtin_amdgcn_readfirstlane(pages[is_page]);
     const int64_t tok0 = blk >= 0 ? (int64_t)blk * bs + is_off : 0;
     is_off += kKC;
     if (is_off == bs) {
@@ -271,6 +243,53 @@ void tree_attn_kernel(AttnParams p) {
       }
     }
   };
+
+  auto issue_chunk = [&](int c, auto stage) {
+    issue_chunk_of(c, __builtin_amdgcn_readfirstlane(pages[is_page]), stage);
+  };
+
+  // The first chunk is on its way before Q, the mask and the page table are asked for, so
+  // a workgroup starts after one memory round trip instead of two (16 prompts of 200 to
+  // 1,800 tokens at 16/8 heads, KV store included: 175.4 -> 169.2 us).
+  using Stage0 = std::integral_constant<int, 0>;
+  using Stage1 = std::integral_constant<int, 1>;
+  if (c0 < c1)
+    issue_chunk_of(c0, __builtin_amdgcn_readfirstlane(page0 < p.bt_stride ? bt[page0] : -1), Stage0{});
+
+  // This split's block-table entries go to LDS once, so the loop reads page ids
+  // without touching the vector-memory counter the DMA pipeline waits on.  Page ids,
+  // mask and Q are loaded together, unconditionally (from a valid row; rows outside
+  // the sequence's are zeroed after), so the compiler waits for them once.
+  const int32_t pg = bt[min(page0 + tid, p.bt_stride - 1)];
+  const bool ld = row_ok && token < p.total_q;
+  const int tok_ld = min(token, p.total_q - 1);
+  uint64_t mbits = 0;
+  if (use_tree) mbits = p.tree_mask[tok_ld];
+  // Q^T fragments (B operand of S^T = K.Q^T): d = 16*s + 8*g + [0..7].
+  uint4 qv[8];
+  {
+    const uint16_t* qrow = p.q + ((int64_t)tok_ld * p.Hq + head) * kD + 8 * g;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) qv[s] = *reinterpret_cast<const uint4*>(qrow + 16 * s);
+  }
+  if (!ld) mbits = 0;
+  if (tid < npages) pages[tid] = page0 + tid < p.bt_stride ? pg : -1;
+  for (int i = tid + W * 64; i < npages; i += W * 64)
+    pages[i] = (page0 + i < p.bt_stride) ? bt[page0 + i] : -1;
+  bf16x8 bq[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    bf16x8 x = __builtin_bit_cast(bf16x8, ld ? qv[s] : make_uint4(0, 0, 0, 0));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = (__bf16)((float)x[e] * p.scale_log2);
+    bq[s] = x;
+  }
+  // Every prologue global load (Q, mask, pages) completes here, before the next LDS-DMA
+  // is queued behind them.
+#pragma unroll
+  for (int s = 0; s < 8; ++s) asm volatile("" : : "v"(bq[s]));
+  asm volatile("" : : "v"(mbits));
+  __syncthreads();
 
   // m_run: the row's reference max (scaled log2 units).  The S chain starts from
   // cinit = -m_ref (m_ref = m_run, or 0 before the row's first visible key), so the
@@ -474,10 +493,7 @@ void tree_attn_kernel(AttnParams p) {
   // One chunk in flight: wait for chunk c, barrier (every wave is done with chunk
   // c-1, whose stage receives chunk c+1), then compute chunk c.  The loop is unrolled
   // by the two ring stages, so each step's stage is a compile-time constant.
-  using Stage0 = std::integral_constant<int, 0>;
-  using Stage1 = std::integral_constant<int, 1>;
   f32x16 sacc[2];
-  if (c0 < c1) issue_chunk(c0, Stage0{});
   for (int c = c0; c < c1; c += 2) {
     wait_vm<0>();
     __syncthreads();
@@ -521,33 +537,88 @@ void tree_attn_kernel(AttnParams p) {
   }
 }
 
-// Merge split partials: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M).  Eight
-// rows per 256-thread workgroup, 32 lanes per row with four elements each (16-byte
-// loads of the fp32 partials).
-constexpr int kCombineRows = 8;
+// Merge split partials: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M).  32 lanes hold
+// a row with four elements each (16-byte loads of the fp32 partials); SP such groups share
+// a row's splits, split s going to group s % SP, and meet in LDS.  A group keeps the
+// partials of kCombineFlight splits in flight with their log-sums, so the merge is a few
+// memory round trips whatever the number of splits: a loop over the splits, one round
+// trip each, took 42 us for 210 splits of 432 rows, 24 us for 119 of 320 and 7 us for 8 of
+// 256 (four groups of a row: 6.4, 5.2 and 4.0 us).
+constexpr int kCombineFlight = 4;
+template <int SP>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ part_o,
                                                       const float* __restrict__ part_lse,
                                                       uint16_t* __restrict__ o, int rows, int nsplit) {
-  const int row = blockIdx.x * kCombineRows + (threadIdx.x >> 5);  // token * Hq + head
-  if (row >= rows) return;
-  const int d = (threadIdx.x & 31) * 4;
-  float M = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, part_lse[(int64_t)s * rows + row]);
+  __shared__ float4 s_num[SP > 1 ? 8 : 1][32];
+  __shared__ float s_m[8], s_den[8];
+  const int grp = threadIdx.x >> 5, l = threadIdx.x & 31, sg = grp % SP;
+  const int row = blockIdx.x * (8 / SP) + grp / SP;  // token * Hq + head
+  const bool valid = row < rows;
+  float m = -INFINITY, den = 0.f;
   float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-  float den = 0.f;
-  if (M != -INFINITY) {
-    for (int s = 0; s < nsplit; ++s) {
-      const float lse = part_lse[(int64_t)s * rows + row];
-      if (lse == -INFINITY) continue;
-      const float w = exp2f(lse - M);
-      const float4 v = *reinterpret_cast<const float4*>(part_o + ((int64_t)s * rows + row) * kD + d);
+  for (int s0 = sg; valid && s0 < nsplit; s0 += SP * kCombineFlight) {
+    float lse[kCombineFlight];
+    float4 v[kCombineFlight];
+#pragma unroll
+    for (int i = 0; i < kCombineFlight; ++i) {
+      const int64_t at = (int64_t)min(s0 + i * SP, nsplit - 1) * rows + row;
+      lse[i] = part_lse[at];
+      v[i] = *reinterpret_cast<const float4*>(part_o + at * kD + l * 4);
+    }
+    float mn = m;
+#pragma unroll
+    for (int i = 0; i < kCombineFlight; ++i) {
+      if (s0 + i * SP >= nsplit) lse[i] = -INFINITY;
+      mn = fmaxf(mn, lse[i]);
+    }
+    if (mn == -INFINITY) continue;
+    const float a = exp2f(m - mn);
+    den *= a;
+    num.x *= a;
+    num.y *= a;
+    num.z *= a;
+    num.w *= a;
+    m = mn;
+#pragma unroll
+    for (int i = 0; i < kCombineFlight; ++i) {
+      if (lse[i] == -INFINITY) continue;
+      const float w = exp2f(lse[i] - mn);
       den += w;
+      num.x += w * v[i].x;
+      num.y += w * v[i].y;
+      num.z += w * v[i].z;
+      num.w += w * v[i].w;
+    }
+  }
+  if constexpr (SP > 1) {
+    s_num[grp][l] = num;
+    if (l == 0) {
+      s_m[grp] = m;
+      s_den[grp] = den;
+    }
+    __syncthreads();
+    if (sg != 0) return;
+    float M = m;
+#pragma unroll
+    for (int g = 1; g < SP; ++g) M = fmaxf(M, s_m[grp + g]);
+    const float a = M == -INFINITY ? 0.f : exp2f(m - M);
+    den *= a;
+    num.x *= a;
+    num.y *= a;
+    num.z *= a;
+    num.w *= a;
+#pragma unroll
+    for (int g = 1; g < SP; ++g) {
+      const float w = M == -INFINITY ? 0.f : exp2f(s_m[grp + g] - M);
+      const float4 v = s_num[grp + g][l];
+      den += w * s_den[grp + g];
       num.x += w * v.x;
       num.y += w * v.y;
       num.z += w * v.z;
       num.w += w * v.w;
     }
   }
+  if (!valid) return;
   uint2 pk;
   if (den > 0.f) {
     pk.x = (uint32_t)f2bf(num.x / den) | ((uint32_t)f2bf(num.y / den) << 16);
@@ -555,7 +626,24 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
   } else {
     pk.x = pk.y = 0u;
   }
-  *reinterpret_cast<uint2*>(o + (int64_t)row * kD + d) = pk;
+  *reinterpret_cast<uint2*>(o + (int64_t)row * kD + l * 4) = pk;
+}
+
+// Groups per row: as many as bring every split's partials in with one or two round trips
+// (8 at most, from 32 splits on more).
+void launch_combine(const AttnParams& p, int rows, hipStream_t s) {
+#define NVX_COMBINE(SP)                                                                      \
+  hipLaunchKernelGGL(combine_kernel<SP>, dim3((rows + 8 / SP - 1) / (8 / SP)), dim3(256), 0, s, \
+                     p.part_o, p.part_lse, p.o, rows, p.nsplit)
+  if (p.nsplit <= kCombineFlight)
+    NVX_COMBINE(1);
+  else if (p.nsplit <= 2 * kCombineFlight)
+    NVX_COMBINE(2);
+  else if (p.nsplit <= 4 * kCombineFlight)
+    NVX_COMBINE(4);
+  else
+    NVX_COMBINE(8);
+#undef NVX_COMBINE
 }
 
 struct Plan {
@@ -709,9 +797,7 @@ int tree_attention_run(const void* q, void* o, const void* k_cache, const void* 
   }
   NVX_LAUNCHED();
   if (pl.nsplit > 1) {
-    const int rows = total_q * num_heads;
-    hipLaunchKernelGGL(combine_kernel, dim3((rows + kCombineRows - 1) / kCombineRows), dim3(256), 0,
-                       s, p.part_o, p.part_lse, (uint16_t*)o, rows, pl.nsplit);
+    launch_combine(p, total_q * num_heads, s);
     NVX_LAUNCHED();
   }
   return NVX_OK;
