@@ -131,12 +131,13 @@ def check(rc):
 
 
 def ptr(t):
-    """Device pointer of a tensor (None -> NULL)."""
-    return None if t is None else c_void_p(t.data_ptr())
+    """Device pointer of a tensor (None -> NULL), as the int a c_void_p argument takes."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(t):
-    return c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """Handle of the current stream of the tensor's device, without a Stream object."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_cuda(*tensors):

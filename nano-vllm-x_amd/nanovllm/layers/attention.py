@@ -99,13 +99,13 @@ def tree_attention(q, k_cache, v_cache, block_tables, cu_seqlens_q, context_lens
     o = torch.empty_like(q) if out is None else out
     L = _C.lib()
     ws_bytes = L.nvx_tree_attention_workspace_size(B, N, max_seqlen_q, max_context_len, Hq, Hkv, D)
-    ws = (_workspace(ws_bytes, q.device, torch.cuda.current_stream(q.device).cuda_stream)
-          if ws_bytes else None)
+    stream = _C.stream_of(q)
+    ws = _workspace(ws_bytes, q.device, stream) if ws_bytes else None
     _C.check(L.nvx_tree_attention(
         _C.ptr(q), _C.ptr(o), _C.ptr(k_cache), _C.ptr(v_cache), _C.ptr(block_tables),
         block_tables.shape[1] if block_tables.dim() == 2 else 1, _C.ptr(cu_seqlens_q),
         _C.ptr(context_lens), _C.ptr(tree_mask), B, N, max_seqlen_q, max_context_len, Hq, Hkv, D,
-        bs, float(scale), _C.ptr(ws), ws_bytes, _C.stream_of(q)))
+        bs, float(scale), _C.ptr(ws), ws_bytes, stream))
     return o
 
 

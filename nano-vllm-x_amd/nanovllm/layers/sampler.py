@@ -85,7 +85,7 @@ def walk_workspace(num_seqs, device, workspace=None):
     if torch.cuda.is_current_stream_capturing():
         return None, 0
     need = _C.lib().nvx_rejection_walk_workspace_size(num_seqs)
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, torch._C._cuda_getCurrentRawStream(device.index))
     ws = _WALK_WS.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.zeros(max(need, _C.lib().nvx_rejection_walk_workspace_size(256)),
