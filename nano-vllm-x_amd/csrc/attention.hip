@@ -540,12 +540,12 @@ void tree_attn_kernel(AttnParams p) {
 // Merge split partials: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M).  32 lanes hold
 // a row with four elements each (16-byte loads of the fp32 partials); SP such groups share
 // a row's splits, split s going to group s % SP, and meet in LDS.  A group keeps the
-// partials of kCombineFlight splits in flight with their log-sums, so the merge is a few
+// partials of FL splits in flight with their log-sums, so the merge is a few
 // memory round trips whatever the number of splits: a loop over the splits, one round
 // trip each, took 42 us for 210 splits of 432 rows, 24 us for 119 of 320 and 7 us for 8 of
 // 256 (four groups of a row: 6.4, 5.2 and 4.0 us).
-constexpr int kCombineFlight = 4;
-template <int SP>
+constexpr int kFlight = 4;
+template <int SP, int FL = kFlight>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ part_o,
                                                       const float* __restrict__ part_lse,
                                                       uint16_t* __restrict__ o, int rows, int nsplit) {
@@ -556,18 +556,18 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
   const bool valid = row < rows;
   float m = -INFINITY, den = 0.f;
   float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int s0 = sg; valid && s0 < nsplit; s0 += SP * kCombineFlight) {
-    float lse[kCombineFlight];
-    float4 v[kCombineFlight];
+  for (int s0 = sg; valid && s0 < nsplit; s0 += SP * FL) {
+    float lse[FL];
+    float4 v[FL];
 #pragma unroll
-    for (int i = 0; i < kCombineFlight; ++i) {
+    for (int i = 0; i < FL; ++i) {
       const int64_t at = (int64_t)min(s0 + i * SP, nsplit - 1) * rows + row;
       lse[i] = part_lse[at];
       v[i] = *reinterpret_cast<const float4*>(part_o + at * kD + l * 4);
     }
     float mn = m;
 #pragma unroll
-    for (int i = 0; i < kCombineFlight; ++i) {
+    for (int i = 0; i < FL; ++i) {
       if (s0 + i * SP >= nsplit) lse[i] = -INFINITY;
       mn = fmaxf(mn, lse[i]);
     }
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
     num.w *= a;
     m = mn;
 #pragma unroll
-    for (int i = 0; i < kCombineFlight; ++i) {
+    for (int i = 0; i < FL; ++i) {
       if (lse[i] == -INFINITY) continue;
       const float w = exp2f(lse[i] - mn);
       den += w;
@@ -632,17 +632,19 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
 // Groups per row: as many as bring every split's partials in with one or two round trips
 // (8 at most, from 32 splits on more).
 void launch_combine(const AttnParams& p, int rows, hipStream_t s) {
-#define NVX_COMBINE(SP)                                                                      \
-  hipLaunchKernelGGL(combine_kernel<SP>, dim3((rows + 8 / SP - 1) / (8 / SP)), dim3(256), 0, s, \
+#define NVX_COMBINE(SP, FL)                                                                  \
+  hipLaunchKernelGGL((combine_kernel<SP, FL>), dim3((rows + 8 / SP - 1) / (8 / SP)), dim3(256), 0, s, \
                      p.part_o, p.part_lse, p.o, rows, p.nsplit)
-  if (p.nsplit <= kCombineFlight)
-    NVX_COMBINE(1);
-  else if (p.nsplit <= 2 * kCombineFlight)
-    NVX_COMBINE(2);
-  else if (p.nsplit <= 4 * kCombineFlight)
-    NVX_COMBINE(4);
+  if (p.nsplit <= 2)
+    NVX_COMBINE(1, 2);
+  else if (p.nsplit <= kFlight)
+    NVX_COMBINE(1, kFlight);
+  else if (p.nsplit <= 2 * kFlight)
+    NVX_COMBINE(2, kFlight);
+  else if (p.nsplit <= 4 * kFlight)
+    NVX_COMBINE(4, kFlight);
   else
-    NVX_COMBINE(8);
+    NVX_COMBINE(8, kFlight);
 #undef NVX_COMBINE
 }
 
@@ -667,10 +669,10 @@ int waves_for(int rows, int max_q) { return rows > 128 && max_q <= 64 ? 8 : 4; }
 // them) must fit the workgroup's LDS page table.
 int max_split_chunks(int block_size) { return ((kMaxSplitPages - 1) * block_size) / kKC; }
 
-// KV splits: enough to fill one round of kTargetWaves waves (at least ~two chunks per
-// split), and at least as many as keep every split within the page table, so a long
-// context is split further rather than refused.  block_size = kKC gives the most
-// splits any allowed page size needs (the workspace size query has no block size).
+// KV splits: enough to fill one round of kTargetWaves waves, and at least as many as keep
+// every split within the page table, so a long context is split further rather than
+// refused.  block_size = kKC gives the most splits any allowed page size needs (the
+// workspace size query has no block size).
 Plan make_plan(int num_seqs, int max_q, int max_ctx, int Hq, int Hkv, int block_size) {
   const int G = Hq / Hkv;
   const int rows = G * (max_q > 0 ? max_q : 1);
@@ -680,7 +682,11 @@ Plan make_plan(int num_seqs, int max_q, int max_ctx, int Hq, int Hkv, int block_
   const int64_t waves = (int64_t)num_seqs * Hkv * pl.nq * pl.waves;
   int ns = (int)((kTargetWaves + waves - 1) / (waves > 0 ? waves : 1));
   const int max_chunks = (max_ctx + kKC - 1) / kKC;
-  const int cap = max(1, max_chunks / 2);
+  // Short contexts: one chunk per split from 8 chunks on, since the merge costs the same
+  // 2 to 3 us for 4 and for 16 splits (one sequence of 701 keys, 16/8 heads: 11 splits
+  // 6.7 + 3.2 us, 5 splits 8.7 + 2.4 us); below, splitting saves less than the merge costs
+  // (4 sequences of 195 keys: 4 splits 6.3 + 2.6 us, one 8.4 us and no second launch).
+  const int cap = max_chunks >= 8 ? max_chunks : max(1, max_chunks / 2);
   if (ns > cap) ns = cap;
   const int per_split = max_split_chunks(block_size);
   const int ns_min = (max_chunks + per_split - 1) / per_split;

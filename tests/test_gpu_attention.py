@@ -248,3 +248,15 @@ def test_random_shapes(dev, case):
     if causal:
         trees = [chain_parents(len(t)) for t in trees]
     run_case(dev, Hq, Hkv, ctx, trees, seed=2000 + case, causal=causal)
+
+
+@pytest.mark.gpu
+# Context lengths in 64-key pages: no split, then every number of splits where the merge
+# changes shape (2, 4, 8 and 16 splits and one more), and more than it keeps in flight at
+# once; the second sequence leaves most of its splits empty, and its rows and the first's
+# do not fill the merge's last workgroup.
+@pytest.mark.parametrize("pages", [1, 4, 6, 8, 9, 16, 17, 32, 33, 70])
+def test_split_merge_edges(dev, pages):
+    rng = np.random.default_rng(pages)
+    trees = [random_tree(5, 2, rng), chain_parents(2)]
+    run_case(dev, 3, 1, [pages * 64 - 5, 1], trees, seed=pages, block_size=64)
