@@ -42,6 +42,7 @@ constexpr int kTileBytes = kKC * kD * 2;        // one K (or V) chunk: 64 rows x
 constexpr int kStageBytes = 2 * kTileBytes;     // K then V
 constexpr int kDmaPerChunk = kStageBytes / 1024;  // 1 KB per wave-wide 16-byte-per-lane load
 constexpr int kTargetWaves = 256 * 8;           // split-KV target: one round of 8 waves per CU
+constexpr int kMaxPacked = 48;                  // sequences of a packed grid (at most 64, one per lane)
 constexpr int kMaxSplitPages = 512;             // block-table entries one KV split may touch
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -60,7 +61,7 @@ struct AttnParams {
   const uint64_t* tree_mask;
   float* part_o;
   float* part_lse;
-  int bt_stride, num_seqs, total_q, Hq, Hkv, G, block_size, nq, nsplit;
+  int bt_stride, num_seqs, total_q, Hq, Hkv, G, block_size, nq, nsplit, packed;
   float scale_log2;
 };
 
@@ -135,25 +136,48 @@ void tree_attn_kernel(AttnParams p) {
   // the chunks of an item adjacent.  Otherwise (tree masks: the chunks of an item do
   // equal work) the chunks and splits of an item are adjacent and grouped by XCD, so
   // they meet in one L2 (64-node trees at 64/8 heads: 309 us against 323 us).
-  const bool heavy_first = p.nq > 1 && p.tree_mask == nullptr;
-  const int logical = heavy_first ? (int)blockIdx.x : remap_xcd(blockIdx.x, gridDim.x);
-  const int split = logical % p.nsplit;
-  int t = logical / p.nsplit;
-  int qc;
-  if (heavy_first) {
-    const int items = (int)(gridDim.x / ((unsigned)p.nsplit * p.nq));  // (sequence, KV head)
-    qc = p.nq - 1 - t / items;
-    t %= items;
+  // Ragged prompts (p.packed): the grid holds only chunks that exist, the longest
+  // sequence's first and each sequence's heaviest first; see the launch.
+  const int lane = threadIdx.x & 63;
+  int split = 0, qc, hk, b, q0, qlen, ctxlen;
+  if (p.packed) {
+    hk = (int)(blockIdx.x % (unsigned)p.Hkv);
+    const int t = (int)(blockIdx.x / (unsigned)p.Hkv);
+    const int sq = min(lane, p.num_seqs - 1);
+    const int my_q0 = p.cu_q[sq], my_len = p.cu_q[sq + 1] - my_q0, my_ctx = p.ctx_lens[sq];
+    const int n = lane < p.num_seqs && my_len > 0 ? (p.G * my_len + W * 32 - 1) / (W * 32) : 0;
+    const int key = n * 64 + 63 - lane;  // order: more chunks first, then the lower index
+    int start = 0;  // chunks of the sequences before this lane's
+    for (int i = 0; i < p.num_seqs; ++i) {
+      const int ki = __builtin_amdgcn_readlane(key, i);
+      start += ki > key ? ki >> 6 : 0;
+    }
+    const uint64_t here = __ballot(t >= start && t < start + n);
+    if (!here) return;  // uniform over the block
+    b = __builtin_ctzll(here);
+    qc = __builtin_amdgcn_readlane(start + n, b) - 1 - t;
+    q0 = __builtin_amdgcn_readlane(my_q0, b);
+    qlen = __builtin_amdgcn_readlane(my_len, b);
+    ctxlen = __builtin_amdgcn_readlane(my_ctx, b);
   } else {
-    qc = t % p.nq;
-    t /= p.nq;
+    const bool heavy_first = p.nq > 1 && p.tree_mask == nullptr;
+    const int logical = heavy_first ? (int)blockIdx.x : remap_xcd(blockIdx.x, gridDim.x);
+    split = logical % p.nsplit;
+    int t = logical / p.nsplit;
+    if (heavy_first) {
+      const int items = (int)(gridDim.x / ((unsigned)p.nsplit * p.nq));  // (sequence, KV head)
+      qc = p.nq - 1 - t / items;
+      t %= items;
+    } else {
+      qc = t % p.nq;
+      t /= p.nq;
+    }
+    hk = t % p.Hkv;
+    b = t / p.Hkv;
+    q0 = p.cu_q[b];
+    qlen = p.cu_q[b + 1] - q0;
+    ctxlen = p.ctx_lens[b];
   }
-  const int hk = t % p.Hkv;
-  const int b = t / p.Hkv;
-
-  const int q0 = p.cu_q[b];
-  const int qlen = p.cu_q[b + 1] - q0;
-  const int ctxlen = p.ctx_lens[b];
   const int base = ctxlen - qlen;
   const int rows_total = p.G * qlen;
   const int row0 = qc * W * 32;
@@ -161,7 +185,7 @@ void tree_attn_kernel(AttnParams p) {
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63, g = lane >> 5, lr = lane & 31;
+  const int g = lane >> 5, lr = lane & 31;
   const int r = row0 + wave * 32 + lr;  // this lane's q row
   const bool row_ok = r < rows_total;
   const bool wave_active = row0 + wave * 32 < rows_total;
@@ -781,7 +805,26 @@ int tree_attention_run(const void* q, void* o, const void* k_cache, const void* 
 
   hipStream_t s = (hipStream_t)stream;
   nvx::TimerScope timer(timed ? NVX_TIMER_TREE_ATTENTION : -1, s);
-  const int64_t nblocks = (int64_t)num_seqs * num_kv_heads * pl.nq * pl.nsplit;
+  int64_t nblocks = (int64_t)num_seqs * num_kv_heads * pl.nq * pl.nsplit;
+  // Causal prompts of unequal lengths: max_seqlen_q sizes num_seqs * nq chunks per KV
+  // head, many of which need not exist.  The chunks that do are at most one per 32 * waves
+  // rows and one more per sequence; where that is fewer, the grid holds those, and a
+  // workgroup finds its chunk among the sequences' (one per lane).  A sequence's chunks
+  // are adjacent and the KV heads of a chunk go to neighbouring workgroups, so the XCDs
+  // share a sequence's K/V in time.  us per call with the plain grid and packed:
+  //   16 prompts of 200 to 1,800 tokens, 16/8 heads  169, 147;  32/8 heads  338, 290
+  //    8 of 500 to 3,500, 32/8   583, 487            4 of 3,000 to 4,000, 16/8   249, 230
+  //   24 of 200 to 1,100, 16/8   104, 95             48 of 50 to 600, 32/8   131, 125
+  //   64 of 17 to 250, 32/8      69, 76: looking through 64 sequences costs a workgroup
+  //   more than its few chunks of keys save, so the line is at 48.
+  p.packed = 0;
+  if (tree_mask == nullptr && pl.nq > 1 && pl.nsplit == 1 && num_seqs <= kMaxPacked) {
+    const int64_t chunks = (int64_t)p.G * total_q / (pl.waves * 32) + num_seqs;
+    if (chunks < (int64_t)num_seqs * pl.nq) {
+      p.packed = 1;
+      nblocks = chunks * num_kv_heads;
+    }
+  }
   NVX_CHECK(nblocks < (1ll << 31), "tree_attention: grid too large");
   const dim3 grid((unsigned)nblocks);
   // One q-row chunk per (sequence, KV head): K/V is streamed once (32 sequences of

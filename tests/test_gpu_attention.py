@@ -6,7 +6,7 @@ import torch
 from nanovllm.layers.attention import tree_attention, Attention
 from nanovllm.spec.tree import chain_parents, random_tree
 from nanovllm.utils.context import set_context, reset_context
-from nanovllm.utils.synthetic import VerifyBatch, randn_bf16
+from nanovllm.utils.synthetic import VerifyBatch, paged_block_tables, randn_bf16
 from oracle import attention as oatt
 
 TOL = 2e-2
@@ -260,3 +260,28 @@ def test_split_merge_edges(dev, pages):
     rng = np.random.default_rng(pages)
     trees = [random_tree(5, 2, rng), chain_parents(2)]
     run_case(dev, 3, 1, [pages * 64 - 5, 1], trees, seed=pages, block_size=64)
+
+
+@pytest.mark.gpu
+# Prompts whose lengths leave most of the launch's chunks empty: lengths on both sides of a
+# chunk (16 tokens of 8 heads) and of a page, empty prompts, equal lengths, a cached prefix;
+# as many sequences as one grid is packed for and one more.  Contexts stay within two key
+# chunks, so no launch is split over the keys.
+@pytest.mark.parametrize("lens,prefix", [
+    ([128, 1, 16, 17, 15, 64, 65], 0), ([0, 128, 0, 3, 3, 128, 0], 0), ([60, 2, 33, 60], 64),
+    ([120] + [5] * 47, 0), ([120] + [5] * 48, 0), ([40, 128] * 24, 0)])
+def test_ragged_prompts(dev, lens, prefix):
+    rng = np.random.default_rng(len(lens))
+    g = torch.Generator().manual_seed(len(lens) + prefix)
+    lens = np.array(lens, np.int32)
+    ends = lens + prefix
+    bt, nblk = paged_block_tables(ends, 64, rng)
+    kc, vc = randn_bf16((nblk, 64, 2, 128), g), randn_bf16((nblk, 64, 2, 128), g)
+    q = randn_bf16((int(lens.sum()), 16, 128), g)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    o = tree_attention(q.to(dev), kc.to(dev), vc.to(dev), torch.from_numpy(bt).to(dev),
+                       torch.from_numpy(cu).to(dev), torch.from_numpy(ends).to(dev), 128 ** -0.5,
+                       None, int(lens.max()), 128)
+    ref = oatt.paged_attention(q.float().numpy(), kc.float().numpy(), vc.float().numpy(), bt, cu, ends,
+                               None, 128 ** -0.5, 64)
+    assert np.abs(o.cpu().float().numpy() - ref).max() < TOL
