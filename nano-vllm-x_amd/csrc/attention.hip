@@ -817,6 +817,8 @@ int tree_attention_run(const void* q, void* o, const void* k_cache, const void* 
   //   24 of 200 to 1,100, 16/8   104, 95             48 of 50 to 600, 32/8   131, 125
   //   64 of 17 to 250, 32/8      69, 76: looking through 64 sequences costs a workgroup
   //   more than its few chunks of keys save, so the line is at 48.
+  // Equal lengths do better in the plain grid, whose order is heaviest first over all
+  // sequences (16 prompts of 1,024 tokens, 16/8: 107, 117).
   p.packed = 0;
   if (tree_mask == nullptr && pl.nq > 1 && pl.nsplit == 1 && num_seqs <= kMaxPacked) {
     const int64_t chunks = (int64_t)p.G * total_q / (pl.waves * 32) + num_seqs;
