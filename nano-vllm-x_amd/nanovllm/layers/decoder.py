@@ -74,10 +74,11 @@ def few_rows_layer(layer, attention_type, mlp_type, positions, hidden, residual,
     mods = layer.__dict__["_modules"]
     sa, mlp, norm_in, norm_post = (mods["self_attn"], mods["mlp"], mods["input_layernorm"],
                                    mods["post_attention_layernorm"])
+    if not (_plain(sa, attention_type) and _plain(mlp, mlp_type)):
+        return None  # replaced modules need not have the submodules read below
     am, mm = sa.__dict__["_modules"], mlp.__dict__["_modules"]
     attn, rope = am["attn"], am["rotary_emb"]
-    if not (_plain(sa, attention_type) and _plain(mlp, mlp_type) and _plain(attn, Attention)
-            and _plain(mm["act_fn"], SiluAndMul)):
+    if not (_plain(attn, Attention) and _plain(mm["act_fn"], SiluAndMul)):
         return None
     Hq, Hkv, D = sa.num_heads, sa.num_kv_heads, sa.head_dim
     down = mm["down_proj"].__dict__["_parameters"].get("weight")

@@ -142,3 +142,32 @@ def test_modules_run_where_something_watches_or_replaces_them(dev):
             assert call() is None
     finally:
         reset_context()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["self_attn", "mlp"])
+def test_replaced_blocks_run_as_modules(dev, name):
+    """A wrapped attention or MLP block has none of the plain one's submodules."""
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, *args):
+            return self.inner(*args)
+
+    layer = _layer(dev)
+    hidden = torch.randn(2, 512).to(torch.bfloat16).to(dev)
+    try:
+        positions, _ = _step(layer, hidden, None, 1, [30, 50], dev, 1)
+        with torch.no_grad():
+            wrapped = Wrapped(getattr(layer, name))
+            setattr(layer, name, wrapped)
+            assert few_rows_layer(layer, Qwen3Attention, Qwen3MLP, positions, hidden, None) is None
+            out, residual = layer(positions, hidden, None)
+            setattr(layer, name, wrapped.inner)
+        with torch.enable_grad():  # the plain layer, module by module
+            want, want_residual = layer(positions, hidden, None)
+        assert torch.equal(out, want) and torch.equal(residual, want_residual)
+    finally:
+        reset_context()
