@@ -217,7 +217,8 @@ int nvx_rejection_sample_tree(const float* target_probs, int64_t p_seq_stride,
  *   draft_tokens int32 or int64 [num_seqs, num_draft]   uniforms fp32 [num_seqs, num_draft]
  *   accepted_len, recovered (-1 when all were accepted), bonus (-1 otherwise) int32 [num_seqs]
  *   out_tokens   int32 [num_seqs, num_draft + 1] (-1 padded)
- * Other arguments as nvx_rejection_sample_tree.
+ * num_draft may be 0 (then draft_probs, draft_tokens and uniforms may be NULL).  Other
+ * arguments as nvx_rejection_sample_tree.
  */
 int nvx_rejection_sample_chain(const float* target_probs, int64_t p_seq_stride,
                                const float* draft_probs, int64_t q_seq_stride, int32_t vocab,

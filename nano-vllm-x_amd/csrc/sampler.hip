@@ -1662,8 +1662,9 @@ extern "C" int nvx_rejection_sample_chain(
   NVX_CHECK(num_draft >= 0 && num_draft < kMaxNodes,
             "rejection_sample_chain: num_draft must be in [0, %d] (got %d)", kMaxNodes - 1, num_draft);
   if (num_seqs == 0) return NVX_OK;
-  NVX_CHECK(target_probs && draft_probs && final_uniforms && accepted_len && recovered && bonus &&
-                out_tokens && (num_draft == 0 || (draft_tokens && uniforms)),
+  // without draft tokens no draft row is read either
+  NVX_CHECK(target_probs && final_uniforms && accepted_len && recovered && bonus && out_tokens &&
+                (num_draft == 0 || (draft_probs && draft_tokens && uniforms)),
             "rejection_sample_chain: null pointer");
   NVX_CHECK(vocab <= kMaxVocab, "rejection_sample_chain: vocab %d exceeds %d", vocab, kMaxVocab);
   uint64_t* ex = nullptr;

@@ -553,3 +553,20 @@ def test_chain_forms(dev, B, k, V, tok_dtype, greedy):
                                      None if flags is None else flags.to(dev, greedy))
         for a, r in zip(out, ref):
             assert a.dtype == torch.int32 and np.array_equal(a.cpu().numpy(), r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,V", [(1, 1003), (3, 512), (9, 32000)])
+def test_chain_without_draft_tokens(dev, B, V):
+    """k = 0: one draw per sequence, the bonus token; nothing of the (empty) draft is read."""
+    g = torch.Generator().manual_seed(V)
+    P = torch.softmax(torch.randn(B, 1, V, generator=g) * 2, -1).to(dev)
+    Uf = torch.rand(B, generator=g)
+    none = torch.zeros(B, 0, device=dev)
+    greedy = torch.arange(B, device=dev) % 2 == 1
+    ref = osamp.rejection_sample_chain(P.cpu().numpy(), np.zeros((B, 0, V)), np.zeros((B, 0)),
+                                       np.zeros((B, 0)), Uf.numpy(), greedy.cpu().numpy())
+    out = rejection_sample_chain(P, torch.zeros(B, 0, V, device=dev), none.long(), none, Uf.to(dev), greedy)
+    for a, r in zip(out, ref):
+        assert np.array_equal(a.cpu().numpy(), r)
+    assert torch.equal(out[2], out[3][:, 0]) and (out[1] == -1).all()
