@@ -68,6 +68,13 @@ def _flags(t, dev):
     return t.to(device=dev, dtype=torch.uint8).contiguous()
 
 
+def _spread(t, rows, cols):
+    """t broadcast to [rows, cols] as assigning it to such a tensor would, contiguous."""
+    while t.dim() > 2 and t.shape[0] == 1:
+        t = t[0]
+    return t.expand(rows, cols).contiguous()
+
+
 _WALK_WS = {}  # (device index, stream) -> zero-filled uint8 tensor, grown on demand
 
 
@@ -327,8 +334,8 @@ def rejection_sample_chain(target_probs, draft_probs, draft_token_ids, uniforms,
     tok = draft_token_ids
     if tok.dtype not in (torch.int32, torch.int64):
         tok = tok.to(torch.int32)
-    tok = tok.to(dev).expand(B, k).contiguous()
-    u = uniforms.to(device=dev, dtype=torch.float32).expand(B, k).contiguous()
+    tok = _spread(tok.to(dev), B, k)
+    u = _spread(torch.as_tensor(uniforms, dtype=torch.float32, device=dev), B, k)
     final_uniforms = final_uniforms.to(torch.float32).contiguous()
     g = None if greedy is None else _flags(greedy, dev)
     # accepted_len, recovered, bonus [B] and tokens [B, k + 1] in one allocation

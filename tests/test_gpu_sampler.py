@@ -570,3 +570,26 @@ def test_chain_without_draft_tokens(dev, B, V):
     for a, r in zip(out, ref):
         assert np.array_equal(a.cpu().numpy(), r)
     assert torch.equal(out[2], out[3][:, 0]) and (out[1] == -1).all()
+
+
+@pytest.mark.gpu
+def test_chain_inputs_broadcast(dev):
+    """Draft tokens and uniforms of any shape that broadcasts to [B, k], and a number as
+    the uniforms of every test."""
+    B, k, V = 3, 4, 512
+    g = torch.Generator().manual_seed(1)
+    P = torch.softmax(torch.randn(B, k + 1, V, generator=g) * 2, -1).to(dev)
+    Q = torch.softmax(torch.randn(B, k, V, generator=g) * 2, -1).to(dev)
+    tok, u = torch.randint(0, V, (B, k), generator=g).to(dev), torch.rand(B, k, generator=g).to(dev)
+    uf = torch.rand(B, generator=g).to(dev)
+
+    def check(t, x, full_t, full_x):
+        got = rejection_sample_chain(P, Q, t, x, uf)
+        want = rejection_sample_chain(P, Q, full_t, full_x, uf)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+    check(tok[None], u[None, None], tok, u)
+    check(tok[0], u[0], tok[0].repeat(B, 1), u[0].repeat(B, 1))
+    check(tok[:, :1], u[:, :1], tok[:, :1].repeat(1, k), u[:, :1].repeat(1, k))
+    check(tok.cpu(), u.cpu().double(), tok, u)
+    check(tok, 0.25, tok, torch.full_like(u, 0.25))
