@@ -92,7 +92,8 @@ def walk_workspace(num_seqs, device, workspace=None):
     if torch.cuda.is_current_stream_capturing():
         return None, 0
     need = _C.lib().nvx_rejection_walk_workspace_size(num_seqs)
-    key = (device.index, torch._C._cuda_getCurrentRawStream(device.index))
+    index = torch.cuda.current_device() if device.index is None else device.index
+    key = (index, torch._C._cuda_getCurrentRawStream(index))
     ws = _WALK_WS.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.zeros(max(need, _C.lib().nvx_rejection_walk_workspace_size(256)),

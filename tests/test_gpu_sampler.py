@@ -11,7 +11,7 @@ from nanovllm import _C
 from nanovllm.layers.sampler import (RejectionSampler, Sampler, rejection_sample_chain,
                                      rejection_sample_tree, rejection_sample_tree_logits,
                                      rejection_sample_tree_logits_lazy, softmax_from_stats,
-                                     softmax_stats, stats_eligible, temperature_softmax)
+                                     softmax_stats, stats_eligible, temperature_softmax, walk_workspace)
 from nanovllm.spec.tree import chain_parents, random_tree
 from oracle import sampler as osamp
 
@@ -593,3 +593,13 @@ def test_chain_inputs_broadcast(dev):
     check(tok[:, :1], u[:, :1], tok[:, :1].repeat(1, k), u[:, :1].repeat(1, k))
     check(tok.cpu(), u.cpu().double(), tok, u)
     check(tok, 0.25, tok, torch.full_like(u, 0.25))
+
+
+@pytest.mark.gpu
+def test_walk_workspace_device_forms(dev):
+    """A device without an index is the current one; one workspace per device and stream."""
+    ws, n = walk_workspace(3, torch.device("cuda"))
+    same, _ = walk_workspace(3, torch.device("cuda", torch.cuda.current_device()))
+    assert ws.data_ptr() == same.data_ptr() and n >= _C.lib().nvx_rejection_walk_workspace_size(3)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert walk_workspace(3, torch.device("cuda"))[0].data_ptr() != ws.data_ptr()
