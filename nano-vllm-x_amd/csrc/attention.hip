@@ -28,6 +28,7 @@
 // visible to node i iff bit m of its tree mask (or m <= i without a mask).
 // With more than one split, partial (o, log2-sum-exp) go to the workspace and a
 // second kernel merges them.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -43,6 +44,7 @@ constexpr int kStageBytes = 2 * kTileBytes;     // K then V
 constexpr int kDmaPerChunk = kStageBytes / 1024;  // 1 KB per wave-wide 16-byte-per-lane load
 constexpr int kTargetWaves = 256 * 8;           // split-KV target: one round of 8 waves per CU
 constexpr int kMaxPacked = 48;                  // sequences of a packed grid (at most 64, one per lane)
+constexpr int64_t kShortPartials = 5120;        // rows of split partials worth single-chunk splits
 constexpr int kMaxSplitPages = 512;             // block-table entries one KV split may touch
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -706,11 +708,21 @@ Plan make_plan(int num_seqs, int max_q, int max_ctx, int Hq, int Hkv, int block_
   const int64_t waves = (int64_t)num_seqs * Hkv * pl.nq * pl.waves;
   int ns = (int)((kTargetWaves + waves - 1) / (waves > 0 ? waves : 1));
   const int max_chunks = (max_ctx + kKC - 1) / kKC;
-  // Short contexts: one chunk per split from 8 chunks on, since the merge costs the same
-  // 2 to 3 us for 4 and for 16 splits (one sequence of 701 keys, 16/8 heads: 11 splits
-  // 6.7 + 3.2 us, 5 splits 8.7 + 2.4 us); below, splitting saves less than the merge costs
+  // Two chunks per split at least.  From 8 chunks on, one per split as long as the merge has
+  // no more than kShortPartials rows of partials to read: it then costs the same 2 to 3 us
+  // for 4 and for 16 splits, while below 8 chunks splitting saves less than the merge costs
   // (4 sequences of 195 keys: 4 splits 6.3 + 2.6 us, one 8.4 us and no second launch).
-  const int cap = max_chunks >= 8 ? max_chunks : max(1, max_chunks / 2);
+  // us per call with half as many splits as chunks and with one each, by rows of partials:
+  //   1 sequence of 700 keys, 32/8 heads (11 x 32 rows)      10.0, 8.6
+  //   1 of 520 keys, 16 nodes, 32/8 (9 x 512)                11.5, 9.8
+  //   4 of 530, 6 nodes, 32/8 (9 x 768)                      11.1, 11.4
+  //   2 of 600, 16 nodes, 32/8 (10 x 1,024)                  11.1, 12.0
+  //   8 of 460, 32 nodes, 16/8 (8 x 4,096)                   15.2, 21.5
+  //   4 of 900, 16 nodes, 64/8 (15 x 4,096)                  20.3, 26.2
+  const int half = max(1, max_chunks / 2);
+  const int64_t merge_rows = std::max<int64_t>(1, (int64_t)num_seqs * max(max_q, 1) * Hq);
+  const int cap = max_chunks >= 8 ? (int)std::max<int64_t>(half, std::min<int64_t>(max_chunks, kShortPartials / merge_rows))
+                                  : half;
   if (ns > cap) ns = cap;
   const int per_split = max_split_chunks(block_size);
   const int ns_min = (max_chunks + per_split - 1) / per_split;

@@ -95,3 +95,23 @@ def test_ops_refuse_cpu_tensors():
     from nanovllm.layers.sampler import temperature_softmax
     with pytest.raises(RuntimeError, match="GPU only"):
         temperature_softmax(torch.zeros(2, 8), torch.ones(2))
+
+
+def test_attention_split_plan():
+    """KV splits per plan, read off the workspace size (fp32 [splits, rows, 128 + 1]): half
+    as many as 64-key chunks where the merge has many rows, one per chunk where it has few."""
+    from nanovllm import _C
+
+    def splits(seqs, nodes, keys, heads, kv_heads):
+        n = _C.lib().nvx_tree_attention_workspace_size(seqs, seqs * nodes, nodes, keys, heads, kv_heads, 128)
+        return n / (seqs * nodes * heads * 129 * 4)
+
+    assert splits(1, 1, 700, 16, 8) == 11
+    assert splits(1, 16, 520, 32, 8) == 9
+    assert splits(4, 16, 900, 64, 8) == 7      # 4,096 rows, 15 chunks
+    assert splits(8, 32, 460, 16, 8) == 4      # 4,096 rows, 8 chunks
+    assert splits(2, 32, 2000, 32, 8) == 16    # 2,048 rows, 32 chunks
+    assert splits(4, 6, 530, 32, 8) == 6       # 768 rows: as many as 5,120 partials allow
+    assert splits(1, 1, 440, 16, 8) == 3       # 7 chunks
+    assert splits(64, 1, 4000, 16, 8) == 0     # one round of waves without splits
+    assert _C.lib().nvx_tree_attention_workspace_size(1, 1, 0, 640, 0, 8, 128) == 0
