@@ -566,10 +566,8 @@ void tree_attn_kernel(AttnParams p) {
 // Merge split partials: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M).  32 lanes hold
 // a row with four elements each (16-byte loads of the fp32 partials); SP such groups share
 // a row's splits, split s going to group s % SP, and meet in LDS.  A group keeps the
-// partials of FL splits in flight with their log-sums, so the merge is a few
-// memory round trips whatever the number of splits: a loop over the splits, one round
-// trip each, took 42 us for 210 splits of 432 rows, 24 us for 119 of 320 and 7 us for 8 of
-// 256 (four groups of a row: 6.4, 5.2 and 4.0 us).
+// partials of FL splits in flight with their log-sums, so the merge takes
+// ceil(splits / (SP * FL)) memory round trips; see launch_combine for the choice.
 constexpr int kFlight = 4;
 template <int SP, int FL = kFlight>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ part_o,
@@ -655,8 +653,24 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
   *reinterpret_cast<uint2*>(o + (int64_t)row * kD + l * 4) = pk;
 }
 
-// Groups per row: as many as bring every split's partials in with one or two round trips
-// (8 at most, from 32 splits on more).
+// Few rows: latency bound, so as many groups per row as bring every split's partials in
+// with one or two round trips.  From 1,024 rows on the workgroups fill the chip by
+// themselves; there one group per row is best (eight rows of a split are then one 4 KB
+// read), with more splits in flight.  us per attention call, (groups, splits in flight):
+//                                        (1,4)  (1,8)  (2,8)  (4,4)  (8,4)
+//   4 sequences of 700 keys, 32/8 heads, 11 splits of 128 rows
+//                                         11.7   11.3   10.4   10.1   10.3
+//   1 of 4,000, 32/8, 63 of 32            23.3   20.0   13.6   13.0   11.2
+//   1 of 3,000, 16 nodes, 32/8, 24 of 512 17.4   16.2   13.3   14.9   14.2
+//   2 of 2,000, 32 nodes, 32/8, 16 of 2,048
+//                                         20.5   19.6   23.3   22.7   22.5
+//   8 of 1,300, 32 nodes, 32/8, 8 of 8,192
+//                                         31.9   31.9   34.1   34.2   34.9
+//   1 of 8,000, 64 nodes, 32/8, 32 of 2,048
+//                                         35.4   33.9   28.7   32.7   32.5
+// (A loop over the splits, one round trip each and one group per row: 12.4, 29.7, 29.3,
+// 27.3, 33.7 and 50.3.)
+constexpr int kMergeRows = 1024;
 void launch_combine(const AttnParams& p, int rows, hipStream_t s) {
 #define NVX_COMBINE(SP, FL)                                                                  \
   hipLaunchKernelGGL((combine_kernel<SP, FL>), dim3((rows + 8 / SP - 1) / (8 / SP)), dim3(256), 0, s, \
@@ -665,6 +679,10 @@ void launch_combine(const AttnParams& p, int rows, hipStream_t s) {
     NVX_COMBINE(1, 2);
   else if (p.nsplit <= kFlight)
     NVX_COMBINE(1, kFlight);
+  else if (rows >= kMergeRows && p.nsplit <= 4 * kFlight)
+    NVX_COMBINE(1, 2 * kFlight);
+  else if (rows >= kMergeRows)
+    NVX_COMBINE(2, 2 * kFlight);
   else if (p.nsplit <= 2 * kFlight)
     NVX_COMBINE(2, kFlight);
   else if (p.nsplit <= 4 * kFlight)

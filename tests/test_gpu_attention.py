@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 import torch
 
+from nanovllm import _C
 from nanovllm.layers.attention import tree_attention, Attention
 from nanovllm.spec.tree import chain_parents, random_tree
 from nanovllm.utils.context import set_context, reset_context
@@ -260,6 +261,22 @@ def test_split_merge_edges(dev, pages):
     rng = np.random.default_rng(pages)
     trees = [random_tree(5, 2, rng), chain_parents(2)]
     run_case(dev, 3, 1, [pages * 64 - 5, 1], trees, seed=pages, block_size=64)
+
+
+@pytest.mark.gpu
+# The same with 1,024 rows to merge and more, at one group per row (up to 16 splits) and at
+# two, and at 1,020 rows; by plan, contexts of 2n chunks take n splits here.
+@pytest.mark.parametrize("pages,tokens", [(10, 64), (12, 64), (16, 64), (18, 64), (32, 64), (34, 64),
+                                          (40, 64), (64, 64), (40, 60)])
+def test_split_merge_many_rows(dev, pages, tokens):
+    rng = np.random.default_rng(pages)
+    trees = [random_tree(tokens, 6, rng), random_tree(64, 6, rng)][:1 if tokens < 64 else 2]
+    ctx = [pages * 64 - 70, 3][:len(trees)]
+    heads = 17 if tokens < 64 else 8
+    n, rows = len(trees), sum(len(t) for t in trees) * heads
+    bytes_ = _C.lib().nvx_tree_attention_workspace_size(n, rows // heads, tokens, pages * 64, heads, 1, 128)
+    assert bytes_ // (rows * 129 * 4) > 4 and (rows >= 1024) == (tokens == 64)
+    run_case(dev, heads, 1, ctx, trees, seed=pages, block_size=64)
 
 
 @pytest.mark.gpu
