@@ -43,7 +43,7 @@ constexpr int kTileBytes = kKC * kD * 2;        // one K (or V) chunk: 64 rows x
 constexpr int kStageBytes = 2 * kTileBytes;     // K then V
 constexpr int kDmaPerChunk = kStageBytes / 1024;  // 1 KB per wave-wide 16-byte-per-lane load
 constexpr int kTargetWaves = 256 * 8;           // split-KV target: one round of 8 waves per CU
-constexpr int kMaxPacked = 48;                  // sequences of a packed grid (at most 64, one per lane)
+constexpr int kMaxPacked = 64;                  // sequences of a packed grid (one per lane)
 constexpr int64_t kShortPartials = 5120;        // rows of split partials worth single-chunk splits
 constexpr int kMaxSplitPages = 512;             // block-table entries one KV split may touch
 
@@ -138,8 +138,9 @@ void tree_attn_kernel(AttnParams p) {
   // the chunks of an item adjacent.  Otherwise (tree masks: the chunks of an item do
   // equal work) the chunks and splits of an item are adjacent and grouped by XCD, so
   // they meet in one L2 (64-node trees at 64/8 heads: 309 us against 323 us).
-  // Ragged prompts (p.packed): the grid holds only chunks that exist, the longest
-  // sequence's first and each sequence's heaviest first; see the launch.
+  // Ragged prompts (p.packed): the grid holds only chunks that exist, heaviest first over
+  // all sequences as well: in descending order of the chunk's index, for equal ones by
+  // sequence; see the launch.
   const int lane = threadIdx.x & 63;
   int split = 0, qc, hk, b, q0, qlen, ctxlen;
   if (p.packed) {
@@ -147,17 +148,34 @@ void tree_attn_kernel(AttnParams p) {
     const int t = (int)(blockIdx.x / (unsigned)p.Hkv);
     const int sq = min(lane, p.num_seqs - 1);
     const int my_q0 = p.cu_q[sq], my_len = p.cu_q[sq + 1] - my_q0, my_ctx = p.ctx_lens[sq];
-    const int n = lane < p.num_seqs && my_len > 0 ? (p.G * my_len + W * 32 - 1) / (W * 32) : 0;
-    const int key = n * 64 + 63 - lane;  // order: more chunks first, then the lower index
-    int start = 0;  // chunks of the sequences before this lane's
-    for (int i = 0; i < p.num_seqs; ++i) {
-      const int ki = __builtin_amdgcn_readlane(key, i);
-      start += ki > key ? ki >> 6 : 0;
+    const int n = lane < p.num_seqs && my_len > 0 ? min((p.G * my_len + W * 32 - 1) / (W * 32), p.nq) : 0;
+    // Chunks of index c or more, over all sequences.
+    auto from = [&](int c) {
+      int x = max(n - c, 0);
+      x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8: lane 15
+      x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // of each row of 16 has its sum
+      x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+      x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+      return __builtin_amdgcn_readlane(x, 15) + __builtin_amdgcn_readlane(x, 31) +
+             __builtin_amdgcn_readlane(x, 47) + __builtin_amdgcn_readlane(x, 63);
+    };
+    if (t >= from(0)) return;                // uniform over the block
+    int lo = 0, hi = p.nq, before = 0;       // from(lo) > t >= from(hi) = before
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1, f = from(mid);
+      if (f > t) {
+        lo = mid;
+      } else {
+        hi = mid;
+        before = f;
+      }
     }
-    const uint64_t here = __ballot(t >= start && t < start + n);
-    if (!here) return;  // uniform over the block
-    b = __builtin_ctzll(here);
-    qc = __builtin_amdgcn_readlane(start + n, b) - 1 - t;
+    qc = lo;
+    // chunk qc of the (t - before)-th sequence that has one
+    const uint64_t level = __ballot(n > qc);
+    const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(level >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((uint32_t)level, 0));
+    b = __builtin_ctzll(__ballot(n > qc && rank == t - before));
     q0 = __builtin_amdgcn_readlane(my_q0, b);
     qlen = __builtin_amdgcn_readlane(my_len, b);
     ctxlen = __builtin_amdgcn_readlane(my_ctx, b);
@@ -838,21 +856,26 @@ int tree_attention_run(const void* q, void* o, const void* k_cache, const void* 
   int64_t nblocks = (int64_t)num_seqs * num_kv_heads * pl.nq * pl.nsplit;
   // Causal prompts of unequal lengths: max_seqlen_q sizes num_seqs * nq chunks per KV
   // head, many of which need not exist.  The chunks that do are at most one per 32 * waves
-  // rows and one more per sequence; where that is fewer, the grid holds those, and a
-  // workgroup finds its chunk among the sequences' (one per lane).  A sequence's chunks
-  // are adjacent and the KV heads of a chunk go to neighbouring workgroups, so the XCDs
-  // share a sequence's K/V in time.  us per call with the plain grid and packed:
-  //   16 prompts of 200 to 1,800 tokens, 16/8 heads  169, 147;  32/8 heads  338, 290
-  //    8 of 500 to 3,500, 32/8   583, 487            4 of 3,000 to 4,000, 16/8   249, 230
-  //   24 of 200 to 1,100, 16/8   104, 95             48 of 50 to 600, 32/8   131, 125
-  //   64 of 17 to 250, 32/8      69, 76: looking through 64 sequences costs a workgroup
-  //   more than its few chunks of keys save, so the line is at 48.
-  // Equal lengths do better in the plain grid, whose order is heaviest first over all
-  // sequences (16 prompts of 1,024 tokens, 16/8: 107, 117).
+  // rows and one more per sequence; where that is well fewer, the grid holds those in the
+  // plain grid's order, and a workgroup finds its chunk among the sequences' (one per
+  // lane).  us per call with the plain grid and packed:
+  //   16 prompts of 200 to 1,800 tokens, 16/8 heads  127, 94;   32/8 heads  235, 178
+  //    8 of 500 to 3,500, 32/8   369, 327            48 of 50 to 600, 32/8   126, 122
+  //   one of 2,048 and 3 of 128, 32/8  108, 50
+  // Finding the chunk costs a workgroup a few tenths of a us, more than few missing chunks
+  // save where chunks are light.  So the line is by the longest prompt's chunks (nq), as
+  // the share of the plain grid that the packed one has (plain us, packed us):
+  //   nq 8    24 prompts of up to 256, 32/8: 82% 31.5, 32.6;  72% 29.6, 27.2
+  //   nq 16   12 of up to 512, 32/8:         81% 38.0, 39.9;  66% 40.3, 31.2
+  //   nq 32   12 of up to 1,024, 32/8:       93% 121.8, 121.9;  88% 119.0, 111.6
+  //   nq 64    4 of up to 2,048, 32/8:       98% 140.5, 142.9;  91% 130.8, 126.8
+  // (The order matters: a whole sequence before the next took 142 us where both grids take
+  // 135, 7 prompts of 2,048 and one of 128 at 16/8 heads.)
   p.packed = 0;
   if (tree_mask == nullptr && pl.nq > 1 && pl.nsplit == 1 && num_seqs <= kMaxPacked) {
     const int64_t chunks = (int64_t)p.G * total_q / (pl.waves * 32) + num_seqs;
-    if (chunks < (int64_t)num_seqs * pl.nq) {
+    const int share = pl.nq >= 64 ? 15 : pl.nq >= 32 ? 14 : 12;  // sixteenths of the plain grid
+    if (chunks * 16 <= (int64_t)num_seqs * pl.nq * share) {
       p.packed = 1;
       nblocks = chunks * num_kv_heads;
     }

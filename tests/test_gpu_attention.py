@@ -302,3 +302,41 @@ def test_ragged_prompts(dev, lens, prefix):
     ref = oatt.paged_attention(q.float().numpy(), kc.float().numpy(), vc.float().numpy(), bt, cu, ends,
                                None, 128 ** -0.5, 64)
     assert np.abs(o.cpu().float().numpy() - ref).max() < TOL
+
+
+def packs(lens, prefix, G, num_seqs, Hkv=2):
+    """The launch's own rule for the packed grid (and that it is not split over the keys)."""
+    waves = 8 if G * max(lens) > 128 and max(lens) <= 64 else 4
+    nq = -(-G * max(lens) // (32 * waves))
+    chunks = G * sum(lens) // (32 * waves) + num_seqs
+    share = 15 if nq >= 64 else 14 if nq >= 32 else 12
+    whole = max(lens) + prefix <= 3 * 64 or num_seqs * Hkv * nq * waves >= 2048
+    return whole and nq > 1 and num_seqs <= 64 and 16 * chunks <= share * num_seqs * nq
+
+
+@pytest.mark.gpu
+# Which grid each set takes is asserted: 8 waves and 4, with a cached prefix and without, as
+# many sequences as lanes and one more, chunks of one sequence only, equal lengths at every
+# level, and just on both sides of the line for short, middling and long prompts.
+@pytest.mark.parametrize("lens,prefix,packed", [
+    ([60, 2, 3, 2, 1, 60, 5, 4], 64, True), ([60, 2, 3, 2, 60, 60, 5, 4], 64, False),
+    ([120, 3, 17, 5], 64, True), ([128, 1, 16, 17, 15, 64, 65], 0, True), ([128] + [0] * 5, 60, True),
+    ([100] + [5] * 63, 0, True), ([100] + [5] * 64, 0, False), ([1, 128, 33] * 21, 7, True),
+    ([512, 512, 512, 500, 480, 400, 300, 90], 0, True), ([512] * 6 + [460, 400], 0, False),
+    ([1030] + [1000, 990, 700], 0, True), ([1030] * 3 + [1000], 0, False)])
+def test_packed_grid(dev, lens, prefix, packed):
+    assert packs(lens, prefix, 8, len(lens)) == packed
+    rng = np.random.default_rng(len(lens))
+    g = torch.Generator().manual_seed(len(lens) + prefix)
+    lens = np.array(lens, np.int32)
+    ends = lens + prefix
+    bt, nblk = paged_block_tables(ends, 64, rng)
+    kc, vc = randn_bf16((nblk, 64, 2, 128), g), randn_bf16((nblk, 64, 2, 128), g)
+    q = randn_bf16((int(lens.sum()), 16, 128), g)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    o = tree_attention(q.to(dev), kc.to(dev), vc.to(dev), torch.from_numpy(bt).to(dev),
+                       torch.from_numpy(cu).to(dev), torch.from_numpy(ends).to(dev), 128 ** -0.5,
+                       None, int(lens.max()), int(ends.max()))
+    ref = oatt.paged_attention(q.float().numpy(), kc.float().numpy(), vc.float().numpy(), bt, cu, ends,
+                               None, 128 ** -0.5, 64)
+    assert np.abs(o.cpu().float().numpy() - ref).max() < TOL
