@@ -159,15 +159,21 @@ void launch_skinny(const void* x, int64_t x_stride, const void* w, void* out, in
 }
 
 // Output columns per workgroup, 8 * NP.  A wider tile reads x fewer times, but a CU takes
-// in only so many bytes at once, so the weights have to be spread over all 256 of them.
-// us per projection, [out, in] features, from few to many columns per workgroup:
-//   [1024, 3072], 8 rows: 5.2 (128 workgroups of 8), 6.5 (64 of 16)
-//   [4096, 12288], 8 rows: 27.5 (512 of 8), 20.6 (256 of 16), 31.4 (128 of 32)
-//   [6144, 4096], 16 rows: 19.3 (768 of 8), 17.5 (384 of 16), 15.3 (192 of 32);
-//                  8 rows: 15.2, 14.2, 14.6
-//   gate/up [12288, 4096], 8 rows: 38.1 (1536 of 8), 34.1 (768 of 16), with 200 MB of weights
-//   gate/up [3072, 1024], 8 rows: 6.1 (384 of 8), 5.7 (192 of 16)
-// hipBLASLt takes 9.1, 20.6, 14.1 (both row counts) and, SiLU-mul not counted, 42.8 and 8.0.
+// in only so many bytes at once, so the weights have to be spread over most of the 256 of
+// them: the widest tile that leaves kBusy workgroups.  us per projection, [out, in]
+// features, with 8, 16 and 32 columns per workgroup and hipBLASLt:
+//   [2048, 6144],  8 rows:  8.3, 11.0, 16.3, 11.2;  16 rows: 11.0, 13.5, 19.5, 11.3
+//   [2304, 9728],  8 rows: 20.4, 16.4, 24.6, 16.1;  16 rows: 28.9, 20.6, 28.8, 16.6
+//   [4096, 9728],  8 rows: 21.4, 17.1, 25.3, 18.7;  16 rows: 29.8, 21.2, 29.8, 19.2
+//   [4608, 4096], 16 rows: 19.5, 17.9, 14.6, 14.2
+//   [6144, 4096], 16 rows: 20.2, 18.5, 15.7, 15.2;   8 rows: 15.0, 15.0, 15.6, 15.2
+//   [4096, 12288], 16 rows: 35.8, 25.4, 37.9, 22.6;  8 rows: 28.9, 21.7, 34.7, 23.4
+// One row is little x to read again: [3072, 9728] 15.2, 15.5; it keeps the narrow tile where
+// the wider one does not reach every CU.  Up to 8 rows, 32 columns gain too little
+// ([5632, 4096] 14.8, 14.4) to lose the smaller sums.  Gate/up, with 8 and 16 columns each:
+//   [12288, 4096], 8 rows: 41.5, 37.2 (hipBLASLt, SiLU-mul not counted: 47.5)
+//   [3072, 1024],  8 rows:  6.2,  5.8 (8.1)
+constexpr int kBusy = 144, kCUs = 256;
 template <int MG>
 void launch_skinny_rows(const void* x, int64_t x_stride, const void* w, void* out, int M, int N, int K,
                         bool silu, hipStream_t s) {
@@ -177,9 +183,9 @@ void launch_skinny_rows(const void* x, int64_t x_stride, const void* w, void* ou
     else
       launch_skinny<MG, 1, true>(x, x_stride, w, out, M, N, K, s);
   } else {
-    if (MG > 1 && N % 32 == 0 && N / 32 >= 192)
+    if (MG > 1 && N % 32 == 0 && N / 32 >= kBusy)
       launch_skinny<MG, 4, false>(x, x_stride, w, out, M, N, K, s);
-    else if (N % 16 == 0 && N / 16 >= 256)
+    else if (N % 16 == 0 && N / 16 >= (M > 1 ? kBusy : kCUs))
       launch_skinny<MG, 2, false>(x, x_stride, w, out, M, N, K, s);
     else
       launch_skinny<MG, 1, false>(x, x_stride, w, out, M, N, K, s);

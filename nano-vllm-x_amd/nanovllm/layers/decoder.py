@@ -19,11 +19,13 @@ from .layernorm import RMSNorm
 
 MAX_ROWS = 32
 
-# Up to 16 rows the library's projections are faster than hipBLASLt's at every size
-# measured (hidden 1024 and 4096), so the call saves launches and GPU time alike.  At 17 to
-# 32 rows re-reading x for every tile of the weights costs more than it saves once the
-# weights are large: hidden 1024, 29 us for the four projections against 38 us (SiLU-mul
-# included); hidden 4096, 120 us against 101 us.
+# Up to 16 rows the call takes less GPU time than the modules at every size measured
+# (hidden 1024 to 5120 replayed as graphs, weights from HBM: 0.46 to 0.91 of the modules'
+# time, though single projections of 9 to 16 rows can be slower than hipBLASLt's), and it
+# saves launches.  At 17 to 32 rows re-reading x for every tile of the weights costs more
+# than that once the weights are large: us per layer of 32 rows, call and modules,
+# hidden 1024 58, 77; 2048 81, 88 (intermediate 8192: 93, 91); 2560 122, 106; 3072 110, 99;
+# 4096 150, 140.
 ROWS_ANY, HIDDEN_ALL_ROWS = 16, 2048
 
 

@@ -36,7 +36,7 @@ def test_validation_errors_are_reported():
 # every tile width, fewer blocks than waves and uneven shares among them.
 @pytest.mark.parametrize("rows", [1, 7, 8, 9, 16, 17, 32])
 @pytest.mark.parametrize("n,k", [(8, 64), (24, 320), (3072, 192), (3080, 64), (4096, 576), (6144, 128),
-                                 (6160, 64)])
+                                 (6160, 64), (2288, 128), (2304, 64), (4576, 64), (4608, 128)])
 @pytest.mark.parametrize("silu", [0, 1])
 def test_skinny_gemm(dev, rows, n, k, silu):
     g = torch.Generator().manual_seed(rows * 7 + n + k)
