@@ -97,9 +97,14 @@ struct WaveTopK {
 // the threshold for the whole workgroup -- the largest over its waves of the k-th largest
 // lane maximum, each a lower bound of the row's k-th largest value -- so of a row's
 // values a few dozen, not a few dozen per wave, are offered to the lists; and every chunk
-// is kUnroll guarded loads in flight, the last one too.
+// is guarded loads in flight together, the last one too.
 // [256, 32000] bf16, k = 8: 11.8 us; a threshold per wave and a tail of single loads
 // took 16.0 us.
+// The row's last chunk has 1, 2 or kUnroll vectors per thread, as many as it needs, and
+// where half the waves hold the whole row, each keeps to its own threshold and the others
+// have nothing to do: [256, 2048] bf16 9.3 us, with kUnroll masked vectors and the common
+// threshold 11.4, a loop of single vectors 9.1.  From half a vector per thread on the common
+// threshold is better ([1, 8192] 8.8 us, 9.6 without).
 template <typename VT, int NT, typename TokT>
 __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict__ logits,
                                                            int64_t stride, int V, int k,
@@ -111,9 +116,11 @@ __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict_
   __shared__ float red[NW];
   __shared__ uint64_t lists[NW * kMaxK];
   const int row = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint4* src = reinterpret_cast<const uint4*>(logits + (int64_t)row * stride);
   const int nvec = V / P;
+  const bool few = nvec <= NT / 2;  // half the waves hold the row
 
   WaveTopK tk;
   tk.k = k;
@@ -123,17 +130,18 @@ __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict_
   // Lane l of wave w reads vectors w*64 + l + t*NT, t = 0, 1, ...; the loop runs on the
   // workgroup's first vector j so that every lane takes every iteration.
   float m = -INFINITY, m2 = -INFINITY, s = 0.f;
-  auto chunk = [&](int j, auto whole) {
+  auto chunk = [&](int j, auto vectors, auto whole) {
+    constexpr int kN = decltype(vectors)::value;
     constexpr bool kWhole = decltype(whole)::value;  // every thread's vectors are in the row
     const int i = j + tid;
-    uint4 w[kUnroll];
+    uint4 w[kN];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
+    for (int u = 0; u < kN; ++u)
       w[u] = nvx::ld_stream(src + (kWhole ? i + u * NT : min(i + u * NT, nvec - 1)));
-    float x[kUnroll][P];
+    float x[kN][P];
     float lm = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < kN; ++u) {
       Tr::expand(w[u], x[u]);
 #pragma unroll
       for (int e = 0; e < P; ++e) {
@@ -150,7 +158,7 @@ __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict_
     if (m != -INFINITY) {
       float a0 = 0.f, a1 = 0.f;
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
+      for (int u = 0; u < kN; ++u)
 #pragma unroll
         for (int e = 0; e < P; e += 2) {
           a0 += __builtin_amdgcn_exp2f(__builtin_fmaf(x[u][e], kLog2e, -m2));
@@ -159,20 +167,33 @@ __global__ __launch_bounds__(NT) void topk_logprobs_kernel(const VT* __restrict_
       s += a0 + a1;
     }
     if (j == 0) {
-      tk.thr0 = nvx::block_max<NT>(wave_kth_largest(lm, k, lane), red);
+      tk.thr0 = wave_kth_largest(lm, k, lane);
+      if (!few) tk.thr0 = nvx::block_max<NT>(tk.thr0, red);
       tk.thr = tk.thr0;
     }
     if (__ballot(lm >= tk.thr)) {
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
+      for (int u = 0; u < kN; ++u)
 #pragma unroll
         for (int e = 0; e < P; ++e)
           tk.offer(x[u][e], (i + u * NT) * P + e, kWhole || i + u * NT < nvec);
     }
   };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  using All = std::integral_constant<int, kUnroll>;
   int j = 0;
-  for (; j + kUnroll * NT <= nvec; j += kUnroll * NT) chunk(j, std::true_type{});
-  if (j < nvec) chunk(j, std::false_type{});
+  for (; j + kUnroll * NT <= nvec; j += kUnroll * NT) chunk(j, All{}, std::true_type{});
+  const int left = nvec - j;
+  if (few) {
+    if (wid * nvx::kWave < nvec) chunk(0, One{}, std::false_type{});  // no barrier inside
+  } else if (left > 2 * NT) {
+    chunk(j, All{}, std::false_type{});
+  } else if (left > NT) {
+    chunk(j, Two{}, std::false_type{});
+  } else if (left > 0) {
+    chunk(j, One{}, std::false_type{});
+  }
 
   const float M = nvx::block_max<NT>(m, red);
   const float part = (m == -INFINITY) ? 0.f : s * __builtin_amdgcn_exp2f(m2 - M * kLog2e);

@@ -95,3 +95,20 @@ def test_chunk_edges(dev, rows, V, dtype):
     x[1, max(0, min(V, 32768) - 8):min(V, 32768)] += 20.0
     x[-1] = 1.5
     check(dev, x.to(dtype), 8)
+
+
+@pytest.mark.gpu
+# Rows that half the waves hold (512 vectors of 16 bytes at 1,024 threads, 128 at 256) and
+# one vector more; one and two vectors per thread and one more; k from one wave's fill to 64.
+@pytest.mark.parametrize("rows,V", [(3, 2048), (3, 2056), (3, 4096), (3, 4104), (3, 8192), (3, 8200),
+                                    (3, 16384), (3, 16392), (1024, 512), (1024, 520), (1024, 1024),
+                                    (1024, 1032), (1024, 2048), (1024, 2056), (1024, 4104)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k", [8, 64])
+def test_short_rows(dev, rows, V, dtype, k):
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(rows, V, generator=g)
+    x[0, -8:] += 20.0
+    x[1, V // 2:] = float("-inf")
+    x[-1] = 1.5
+    check(dev, x.to(dtype), k)
