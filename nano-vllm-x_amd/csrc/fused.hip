@@ -25,9 +25,11 @@ __device__ __forceinline__ float rbf(float x) { return bf(f2bf(x)); }  // round 
 // add:   s = x + r (fp32); r_out = bf16(s); y from s as above.
 // A decode step's few rows are bound by latency, not bytes: every load, the weight's too,
 // is in flight before the sum of squares is reduced, and a row takes as many threads as it
-// has pieces (kPer pieces each at most).  Add+RMSNorm, back to back: [8, 4096] 4.2 ->
-// 4.05 us, [1, 1024] 2.8 -> 2.65 us, [16384, 1024] 26.5 -> 23.1 us against one 256-thread
-// kernel that asked for the weight after the reduction.
+// has pieces (kPer pieces each at most).  Add+RMSNorm, back to back: [8, 4096] 4.5 ->
+// 3.5 us, [1, 1024] 3.1 -> 2.95 us, [16384, 1024] 25.8 -> 23.1 us against one 256-thread
+// kernel that asked for the weight after the reduction.  That kernel is ahead at about
+// 1,024 rows of 5,120 to 6,144 with a residual ([1024, 5120] 9.8, here 10.4), and behind at
+// fewer and more rows ([256, 5120] 6.3, 5.1; [4096, 8192] 44.8, 42.1).
 constexpr int kNormMaxHidden = 8192;
 template <int NT, int kPer>
 __global__ __launch_bounds__(NT) void rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
@@ -245,10 +247,16 @@ extern "C" int nvx_rmsnorm(const void* x, int64_t x_row_stride, const void* resi
   hipLaunchKernelGGL((rmsnorm_kernel<NT, PER>), dim3(num_rows), dim3(NT), 0, s, (const uint16_t*)x, \
                      x_row_stride, (const uint16_t*)residual, (uint16_t*)residual_out,          \
                      (const uint16_t*)weight, (uint16_t*)out, hidden, eps)
+  // 2,049 to 4,096: with a residual, a piece per thread (us with 256 threads of two and 512 of
+  // one: [1024, 4096] 8.45, 7.95; [4096, 3072] 20.2, 18.8; [16384, 4096] 96.8, 92.3), unless
+  // many rows leave a quarter of the threads idle ([16384, 2560] 61.6, 64.1); without a
+  // residual, two pieces per thread stream many rows better ([16384, 4096] 41.2, 46.1).
   if (hidden <= 128 * 8)
     NVX_NORM(128, 1);
   else if (hidden <= 256 * 8)
     NVX_NORM(256, 1);
+  else if (hidden <= 512 * 8 && residual && (hidden > 384 * 8 || num_rows <= 8192))
+    NVX_NORM(512, 1);
   else if (hidden <= 512 * 8)
     NVX_NORM(256, 2);
   else

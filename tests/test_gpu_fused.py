@@ -50,6 +50,27 @@ def test_rmsnorm_plain_and_add(dev, H):
     assert d.max() <= 2 and d.float().mean() < 0.05
 
 
+@pytest.mark.gpu
+# Every thread count and pieces per thread of the launch: the last size of each, the next
+# one up, the smallest and the largest; odd row counts, with a padded row stride.
+@pytest.mark.parametrize("H,N", [(H, N) for H in (8, 1024, 1032, 2048, 2056, 4096, 4104, 5120, 8184, 8192)
+                                 for N in (1, 5)] + [(3072, 8193), (3080, 8193)])
+def test_rmsnorm_launch_edges(dev, H, N):
+    g = torch.Generator().manual_seed(H + N)
+    x = torch.randn(N, H + 8, generator=g).to(torch.bfloat16)
+    r = torch.randn(N, H, generator=g).to(torch.bfloat16)
+    w = (1 + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16)
+    xd = x.to(dev)[:, :H]
+    y = rms_norm(xd, w.to(dev), 1e-6).cpu()
+    y2, r2 = rms_norm(xd, w.to(dev), 1e-6, r.to(dev))
+    ey, er = ref_rms(x[:, :H], w, 1e-6, r)
+    assert torch.equal(r2.cpu(), er)
+    # as above: a 1-ulp difference in rsqrt can surface as 2 ulps, rarely
+    for got, want in ((y, ref_rms(x[:, :H], w, 1e-6)), (y2.cpu(), ey)):
+        d = ulps(got, want)
+        assert d.max() <= 2 and (d > 0).float().mean() < max(0.05, 2 / d.numel())
+
+
 def ref_rope(x, pos, base=1000000.0):
     """NeoX rotate-half RoPE in fp32 (reference rotary_embedding.py:6-14), with the
     angles computed in float64 from the definition a = p * base^(-2j/D)."""
