@@ -10,7 +10,7 @@ from nanovllm import _C
 from nanovllm.layers.decoder import few_rows_layer
 from nanovllm.models.qwen3 import Qwen3Attention, Qwen3DecoderLayer, Qwen3MLP, random_init_
 from nanovllm.spec.tree import ancestor_masks, random_tree
-from nanovllm.utils.context import reset_context, set_context
+from nanovllm.utils.context import get_context, reset_context, set_context
 from nanovllm.utils.synthetic import paged_block_tables, slots_for
 
 
@@ -79,15 +79,18 @@ def _step(layer, hidden, residual, nodes, ctx, dev, seed):
     return t(np.concatenate([c + np.arange(nodes) for c in ctx]), np.int64), cache
 
 
-def _layer(dev):
+def _layer(dev, hidden=512, inter=1536, qk_norm=True):
     from transformers import Qwen3Config
-    cfg = Qwen3Config(hidden_size=512, intermediate_size=1536, num_hidden_layers=1,
+    cfg = Qwen3Config(hidden_size=hidden, intermediate_size=inter, num_hidden_layers=1,
                       num_attention_heads=4, num_key_value_heads=2, head_dim=128, vocab_size=512,
                       max_position_embeddings=4096, rope_theta=1000000, rms_norm_eps=1e-6,
                       hidden_act="silu", attention_bias=False)
     torch.set_default_dtype(torch.bfloat16)  # the rotary table stays fp32
     try:
         layer = Qwen3DecoderLayer(cfg)
+        if not qk_norm:
+            layer.self_attn = Qwen3Attention(hidden, 4, 2, max_position=4096, head_dim=128,
+                                             rope_theta=1000000, qk_norm=False)
     finally:
         torch.set_default_dtype(torch.float32)
     return random_init_(layer.to(dev), std=0.05)
@@ -169,5 +172,62 @@ def test_replaced_blocks_run_as_modules(dev, name):
         with torch.enable_grad():  # the plain layer, module by module
             want, want_residual = layer(positions, hidden, None)
         assert torch.equal(out, want) and torch.equal(residual, want_residual)
+    finally:
+        reset_context()
+
+
+@pytest.mark.gpu
+# As serving runs every layer after the first: the residual stream between the norms stays
+# in the call's scratch (no aux list).  Decode, tree and prefill contexts (there max_seqlen_k
+# gives the longest context and a mask is dropped), layers with and without q/k norm.
+@pytest.mark.parametrize("ctx,nodes,prefill,qk_norm", [
+    ([5, 700, 90], 1, False, True), ([40, 0, 513, 64], 5, False, True), ([40, 0, 513], 5, False, False),
+    ([0, 300], 16, True, True), ([7], 9, True, False)])
+def test_layer_without_aux(dev, ctx, nodes, prefill, qk_norm):
+    layer, N = _layer(dev, qk_norm=qk_norm), len(ctx) * nodes
+    g = torch.Generator().manual_seed(N)
+    hidden, residual = (torch.randn(N, 512, generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    got = []
+    try:
+        for grad in (False, True):  # gradients: module by module
+            positions, cache = _step(layer, hidden, residual, nodes, ctx, dev, 3)
+            c = get_context()
+            if prefill:
+                set_context(True, cu_seqlens_q=c.cu_seqlens_q, max_seqlen_q=nodes,
+                            max_seqlen_k=c.max_context_len, slot_mapping=c.slot_mapping,
+                            context_lens=c.context_lens, block_tables=c.block_tables,
+                            tree_mask=c.tree_mask)
+            before, slots = cache.clone(), get_context().slot_mapping.long()
+            with torch.set_grad_enabled(grad):
+                assert (few_rows_layer(layer, Qwen3Attention, Qwen3MLP, positions, hidden, residual)
+                        is None) == grad
+                out, res = layer(positions, hidden, residual)
+            got.append((out.detach(), res.detach(), cache.view(2, -1, 256)[:, slots]))
+            kept = torch.ones(cache[0].numel() // 256, dtype=torch.bool, device=dev)
+            kept[slots] = False
+            assert torch.equal(cache.view(2, -1, 256)[:, kept], before.view(2, -1, 256)[:, kept])
+    finally:
+        reset_context()
+    for a, b in zip(got[0][:2], got[1][:2]):  # a dozen roundings to bf16, as above
+        assert ((a.double() - b.double()).norm() / b.double().norm()) < 1e-2
+    # each new K and V row (both heads): a projection, the norm and the rotation, three
+    # roundings to bf16 after sums in another order
+    a, b = got[0][2].double(), got[1][2].double()
+    assert ((a - b).norm(dim=2) <= 1e-2 * b.norm(dim=2)).all()
+
+
+@pytest.mark.gpu
+def test_rows_the_call_leaves_to_the_modules(dev):
+    """17 to 32 rows above hidden 2,048, and a call under autocast."""
+    try:
+        with torch.no_grad():
+            for hidden, rows, used in ((2048, 32, True), (2112, 16, True), (2112, 17, False)):
+                layer = _layer(dev, hidden, 256)
+                x = torch.randn(rows, hidden, device=dev).to(torch.bfloat16)
+                positions, _ = _step(layer, x, None, 1, [30] * rows, dev, 1)
+                call = lambda: few_rows_layer(layer, Qwen3Attention, Qwen3MLP, positions, x, None)  # noqa: E731
+                assert (call() is not None) == used
+                with torch.autocast("cuda", dtype=torch.bfloat16):
+                    assert call() is None
     finally:
         reset_context()
