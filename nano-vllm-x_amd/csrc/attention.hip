@@ -742,24 +742,30 @@ Plan make_plan(int num_seqs, int max_q, int max_ctx, int Hq, int Hkv, int block_
   pl.waves = waves_for(rows, max_q);
   pl.nq = (rows + pl.waves * 32 - 1) / (pl.waves * 32);
   const int64_t waves = (int64_t)num_seqs * Hkv * pl.nq * pl.waves;
-  int ns = (int)((kTargetWaves + waves - 1) / (waves > 0 ? waves : 1));
   const int max_chunks = (max_ctx + kKC - 1) / kKC;
-  // Two chunks per split at least.  From 8 chunks on, one per split as long as the merge has
-  // no more than kShortPartials rows of partials to read: it then costs the same 2 to 3 us
-  // for 4 and for 16 splits, while below 8 chunks splitting saves less than the merge costs
-  // (4 sequences of 195 keys: 4 splits 6.3 + 2.6 us, one 8.4 us and no second launch).
-  // us per call with half as many splits as chunks and with one each, by rows of partials:
+  int ns = (int)((kTargetWaves + waves - 1) / (waves > 0 ? waves : 1));
+  ns = min(ns, max(1, max_chunks / 2));  // about two chunks per split
+  // Fewer chunks per split from 8 chunks on, where that stays within one round of waves and
+  // the merge has no more than kShortPartials rows of partials to read: it then costs the
+  // same 2 to 3 us for 4 and for 16 splits, while below 8 chunks splitting saves less than
+  // the merge costs (4 sequences of 195 keys: 4 splits 6.3 + 2.6 us, one 8.4 us and no
+  // second launch).  us per call with half as many splits as chunks and with more, by rows
+  // of partials:
   //   1 sequence of 700 keys, 32/8 heads (11 x 32 rows)      10.0, 8.6
   //   1 of 520 keys, 16 nodes, 32/8 (9 x 512)                11.5, 9.8
   //   4 of 530, 6 nodes, 32/8 (9 x 768)                      11.1, 11.4
   //   2 of 600, 16 nodes, 32/8 (10 x 1,024)                  11.1, 12.0
   //   8 of 460, 32 nodes, 16/8 (8 x 4,096)                   15.2, 21.5
   //   4 of 900, 16 nodes, 64/8 (15 x 4,096)                  20.3, 26.2
-  const int half = max(1, max_chunks / 2);
+  //   12 of 565, 2 nodes, 32/8 (6 x 768, 1.1 rounds)         13.7, 16.4
+  //   9 of 597, 32/8 (8 x 288, of which 5 not empty)         14.0, 15.8
   const int64_t merge_rows = std::max<int64_t>(1, (int64_t)num_seqs * max(max_q, 1) * Hq);
-  const int cap = max_chunks >= 8 ? (int)std::max<int64_t>(half, std::min<int64_t>(max_chunks, kShortPartials / merge_rows))
-                                  : half;
-  if (ns > cap) ns = cap;
+  const int most = (int)std::min<int64_t>({max_chunks, kShortPartials / merge_rows,
+                                           kTargetWaves / std::max<int64_t>(1, waves)});
+  if (max_chunks >= 8 && most > ns) {
+    const int per = (max_chunks + most - 1) / most;
+    if (per < (max_chunks + ns - 1) / ns) ns = (max_chunks + per - 1) / per;
+  }
   const int per_split = max_split_chunks(block_size);
   const int ns_min = (max_chunks + per_split - 1) / per_split;
   if (ns < ns_min) ns = ns_min;

@@ -111,7 +111,9 @@ def test_attention_split_plan():
     assert splits(4, 16, 900, 64, 8) == 7      # 4,096 rows, 15 chunks
     assert splits(8, 32, 460, 16, 8) == 4      # 4,096 rows, 8 chunks
     assert splits(2, 32, 2000, 32, 8) == 16    # 2,048 rows, 32 chunks
-    assert splits(4, 6, 530, 32, 8) == 6       # 768 rows: as many as 5,120 partials allow
+    assert splits(4, 6, 530, 32, 8) == 5       # 768 rows, 9 chunks: 5,120 partials allow two a split
+    assert splits(12, 2, 567, 32, 8) == 5      # one round of waves allows two a split
+    assert splits(9, 1, 598, 32, 8) == 5       # 10 chunks: seven splits would leave two empty
     assert splits(1, 1, 440, 16, 8) == 3       # 7 chunks
     assert splits(64, 1, 4000, 16, 8) == 0     # one round of waves without splits
     assert _C.lib().nvx_tree_attention_workspace_size(1, 1, 0, 640, 0, 8, 128) == 0
